@@ -168,10 +168,11 @@ class _Model:
             os.unlink(path)
         if not self.h:
             raise RuntimeError(capi.last_error())
+        self.sync = torch.cuda.synchronize
 
     def __del__(self):
         if getattr(self, "h", None):
-            torch.cuda.synchronize()
+            self.sync()
             self.lib.acfun_model_destroy(self.h)
 
 
