@@ -52,6 +52,12 @@ struct G32Conv {
 constexpr int g32_stage(int BM, int BN, int KC) { return BM * KC + KC * BN; }   // floats
 constexpr int g32_vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0F70; }
 
+// 16 bytes per lane from rsrc at byte offset voff (per lane) + soff (scalar)
+// to LDS: lane l's at lds + 16 l.
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rsrc, float* lds, unsigned voff, unsigned soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void32*)lds, 16, voff, soff, 0, 0);
+}
+
 template <int BM, int BN, int NST, bool CONV, int KS, int KC>
 __global__ __launch_bounds__(256 * KS) void k_gemm32(const float* __restrict__ A,
                                                 const float* __restrict__ B,
@@ -111,8 +117,6 @@ __global__ __launch_bounds__(256 * KS) void k_gemm32(const float* __restrict__ A
     // the quad this lane's slot holds (the swizzle is the same for every t:
     // 4 RPI t is a multiple of 16)
     const int aq = KC == 64 ? (lane & 15) ^ (arow & 15) : (lane & 7) ^ ((arow >> 1) & 7);
-    const unsigned av = (unsigned)(arow * lda + 4 * aq) * 4u;
-    const unsigned astep = 4u * RPI * lda * 4u;            // 4 RPI rows per t
     // CONV: per row t, the byte offset of channel quad aq of tap (0, 0) and the
     // in-image taps as bits kh*8 + kw (KH, KW <= 8)
     int cbase[AIT];
@@ -141,43 +145,63 @@ __global__ __launch_bounds__(256 * KS) void k_gemm32(const float* __restrict__ A
             }
         }
     }
-    bool bok[BIT];
-    unsigned bv[BIT];
+    // Lane byte offsets of the items at k = 0 (CONV: of the current tap), kOOB
+    // outside the operand; a chunk adds one scalar offset per operand, so it
+    // costs no address VALU, which fp32 MFMA cannot overlap (1024^3: 22.8 ->
+    // 21.8 us; conv 3x3/2 28 x 28 x 256, batch 16: 51.9 -> 47.2).  Only a chunk
+    // that ends past K masks its lanes.
+    unsigned av[AIT], bv[BIT];
+#pragma unroll
+    for (int t = 0; t < AIT; ++t)
+        av[t] = CONV ? kOOB : (unsigned)((arow + 4 * RPI * t) * lda + 4 * aq) * 4u;
 #pragma unroll
     for (int t = 0; t < BIT; ++t) {
         const int slot = 64 * (wl + 4 * t) + lane;
         const int krow = slot / BQ;
         const int q = (slot % BQ) ^ ((krow & (KC / 2)) ? 8 : 0);   // quad q of k row r: slot q ^ 8[r >= KC/2]
-        bok[t] = n0 + 4 * q < N;
-        bv[t] = (unsigned)(krow * ldb + n0 + 4 * q) * 4u;
+        bv[t] = n0 + 4 * q < N ? (unsigned)(krow * ldb + n0 + 4 * q) * 4u : kOOB;
     }
-    const bool kragged = (K & (KC - 1)) != 0;
+    int kh = 0, kw = 0, icc = kg * KC, tap = -1;       // CONV: tap and channel of the next chunk issued
 
-    // Every variable part of an address is in the per-lane offset (which the
-    // buffer range check covers); the scalar offset stays 0.
-    auto issue = [&](int t, int c, float* st) {            // item t of (local) chunk c into stage st
+    auto issue = [&](int c, float* st) {               // (local) chunk c, in order, into stage st
         const int k0 = (KS * c + kg) * KC;
-        if (t < AIT) {
-            unsigned v;
-            if (KS > 1 && k0 >= K) {
-                v = kOOB;                                   // a group's padding chunk: zeros
-            } else if (CONV) {
-                // a chunk lies in one tap (Cin % 64 == 0): wave-uniform
-                const int tap = k0 / cv.Cin, ic0 = k0 - tap * cv.Cin;
-                const int kh = tap / cv.KW, kw = tap - kh * cv.KW;
-                const bool ok = (cmask[t] >> (kh * 8 + kw)) & 1ull;
-                v = ok ? (unsigned)(cbase[t] + ((kh * cv.W + kw) * cv.Cin + ic0) * 4) : kOOB;
-            } else {
-                v = av + (unsigned)k0 * 4u + (unsigned)t * astep;
-                if (kragged && k0 + 4 * aq >= K) v = kOOB;
+        st += wl * 256;
+        if (k0 + KC <= K) {
+            unsigned sa = (unsigned)k0 * 4u;
+            if (CONV) {                                 // a chunk lies in one tap (Cin % 64 == 0)
+                while (icc >= cv.Cin) {
+                    icc -= cv.Cin;
+                    if (++kw == cv.KW) { kw = 0; ++kh; }
+                }
+                if (kh * 8 + kw != tap) {
+                    tap = kh * 8 + kw;
+                    const int to = (kh * cv.W + kw) * cv.Cin * 4;
+#pragma unroll
+                    for (int t = 0; t < AIT; ++t)
+                        av[t] = (cmask[t] >> tap) & 1ull ? (unsigned)(cbase[t] + to) : kOOB;
+                }
+                sa = (unsigned)icc * 4u;
+                icc += KS * KC;
             }
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, (lds_void32*)(st + (wl + 4 * t) * 256),
-                                                     16, v, 0, 0, 0);
-        } else {
-            const int tt = t - AIT;
-            const unsigned v = bok[tt] && k0 < K ? bv[tt] + (unsigned)k0 * ldb * 4u : kOOB;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                bres, (lds_void32*)(st + SB + (wl + 4 * tt) * 256), 16, v, 0, 0, 0);
+            const unsigned sb = (unsigned)k0 * ldb * 4u;
+#pragma unroll
+            for (int t = 0; t < AIT; ++t)
+                dma16(ares, st + t * 1024, av[t], sa);
+#pragma unroll
+            for (int t = 0; t < BIT; ++t)
+                dma16(bres, st + SB + t * 1024, bv[t], sb);
+        } else {                                        // K's ragged end, or a group's padding chunk
+#pragma unroll
+            for (int t = 0; t < AIT; ++t) {
+                const unsigned v = !CONV && k0 + 4 * aq < K ? av[t] + (unsigned)k0 * 4u : kOOB;
+                dma16(ares, st + t * 1024, v, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < BIT; ++t) {
+                const int krow = (64 * (wl + 4 * t) + lane) / BQ;
+                const unsigned v = k0 + krow < K ? bv[t] + (unsigned)k0 * ldb * 4u : kOOB;   // kOOB stays past the end
+                dma16(bres, st + SB + t * 1024, v, 0);
+            }
         }
     };
 
@@ -236,10 +260,7 @@ __global__ __launch_bounds__(256 * KS) void k_gemm32(const float* __restrict__ A
     float* const smg = sm + kg * NST * STAGE;           // this group's stages
 #pragma unroll
     for (int c0 = 0; c0 < AHEAD; ++c0) {
-        if (c0 < nch) {
-#pragma unroll
-            for (int t = 0; t < ITEMS; ++t) issue(t, c0, smg + c0 * STAGE);
-        }
+        if (c0 < nch) issue(c0, smg + c0 * STAGE);
     }
 
     // Software pipeline per chunk c (operands in registers):
@@ -295,10 +316,7 @@ __global__ __launch_bounds__(256 * KS) void k_gemm32(const float* __restrict__ A
                 for (int j = 0; j < FN; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][s >> 2][s & 3], bb[j][s],
                                                                      acc[i][j], 0, 0, 0);
-            if (more && s == 0) {                  // its stage was read before this chunk
-#pragma unroll
-                for (int t = 0; t < ITEMS; ++t) issue(t, c + AHEAD, NA);
-            }
+            if (more && s == 0) issue(c + AHEAD, NA);   // its stage was read before this chunk
         }
         f4g al[FM];
         float bl[FN][DEFER];
@@ -422,25 +440,31 @@ __global__ __launch_bounds__(256 * KS) void k_gemm32(const float* __restrict__ A
 // leaves a tile's load latency and epilogue exposed: each workgroup runs a
 // list of 64 x 64 tiles back to back, and one DMA stream of (tile, chunk)
 // items runs NST - 1 chunks ahead of the MFMAs across tile boundaries, so
-// the next tile's operands load during the current tile's last chunks and
-// its epilogue.  K in chunks of 32 (the KC = 32 stage layouts above), NST
-// stages of 16 KB, three workgroups per CU.  Tiles: XCD x = blockIdx % 8 owns
-// a contiguous run of k_gemm32's tile order, which its workgroups take round
-// robin.  Every iteration issues the same number of DMA loads (items past
-// the workgroup's last chunk are issued out of range and write zeros to a
-// stage no chunk reads again), so every wait of the loop is the same.
-// Epilogue: the waves write the tile's sums into the stage of its last chunk
-// (every wave has read it), then thread t forms quad t % 16 of rows t/16 +
-// 16i: + bias, + the fused residual, the activation, one 16-byte store (rows
-// and quads past M and N element by element).  Per output the arithmetic is
-// k_gemm32's: the chunk sums in k order, then fl(fl(sum + bias) + res).
+// the next tile's operands load during the current tile's last chunks.  K in
+// chunks of 32 (the KC = 32 stage layouts above), NST stages of 16 KB, four
+// workgroups per CU.  Tiles: XCD x = blockIdx % 8 owns a contiguous run of
+// k_gemm32's tile order, which its workgroups take round robin.  Every
+// iteration issues the same number of DMA loads (past the workgroup's last
+// chunk out of range: zeros to a stage no chunk reads again).
+//
+// What bounds it: fp32 MFMA and VALU share a SIMD's issue, and the four waves
+// of a SIMD hide one another's latencies only while none of them waits for
+// long.  So a chunk carries no address arithmetic (per-tile lane offsets plus
+// one scalar offset per operand), and a finished tile neither goes through LDS
+// nor makes the next chunk's wait include its stores: its sums move to
+// registers and are stored behind the next chunk's DMA, which that chunk's
+// wait does not cover.  Before / after, batch-64 layer shapes: conv 3x3/2
+// 56 x 56 x 128 -> 128 155 / 136 us (109 TFLOP/s), GEMM 4096^3 1,106 / 993 us
+// (138 TFLOP/s), 200704 x 256 x 64 100 / 84 us, 12544 x 1024 x 256 67 / 58 us.
+// Per output the arithmetic is k_gemm32's: the chunk sums in k order, then
+// fl(fl(sum + bias) + res).
 template <int NST, bool CONV>
-__global__ __launch_bounds__(256) void k_gemm32p(const float* __restrict__ A,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_gemm32p(const float* __restrict__ A,
                                                  const float* __restrict__ B,
                                                  float* __restrict__ C,
                                                  const float* __restrict__ bias,
                                                  const float* __restrict__ res, int M, int N, int K,
-                                                 int lda, int ldb, int ldc, int ldr, int act, int vec,
+                                                 int lda, int ldb, int ldc, int ldr, int act,
                                                  unsigned a_bytes, G32Conv cv) {
     constexpr int BM = 64, BN = 64, KC = 32;
     constexpr int STAGE = g32_stage(BM, BN, KC);        // 4096 floats
@@ -501,72 +525,101 @@ __global__ __launch_bounds__(256) void k_gemm32p(const float* __restrict__ A,
         bq4[t] = 4 * ((slot % BQ) ^ ((bkr[t] & (KC / 2)) ? 8 : 0));
     }
     const bool kragged = (K & (KC - 1)) != 0;
-    // issue cursor: tile ik of this workgroup, chunk ic; its rows' descriptors
-    int ik = 0, ic = 0, in0 = 0;
-    unsigned arowoff[AIT];                              // plain: byte offset of the row (kOOB past M)
-    int cbase[AIT];                                     // CONV: tap-(0,0) offset, in-image taps
-    unsigned long long cmask[AIT];
+    // Issue cursor: tile ik of this workgroup, chunk ic.  A lane's byte offsets
+    // (va, vb; kOOB for rows, columns and taps outside the operand) change per
+    // tile (CONV: also per tap); the chunk's advance is one scalar offset per
+    // operand, so a chunk costs the SIMD no VALU, which fp32 MFMA cannot
+    // overlap.  Once the list is done every offset is kOOB: the loads go on,
+    // writing zeros to a stage no chunk reads.
+    int ik = 0, ic = 0;
+    unsigned va0, va1, vb0, vb1;
+    unsigned sa = 0, sb = 0;                            // scalar byte offsets of the chunk
+    // offsets within the tile at (0, 0)
+    const unsigned arel = 4 * aq < K ? (unsigned)(arow * lda + 4 * aq) * 4u : kOOB;
+    const unsigned brel0 = bkr[0] < K ? (unsigned)(bkr[0] * ldb + bq4[0]) * 4u : kOOB;
+    const unsigned brel1 = bkr[1] < K ? (unsigned)(bkr[1] * ldb + bq4[1]) * 4u : kOOB;
+    // the last four tiles set up: the epilogue's is at most three behind
+    int qm0 = 0, qm1 = 0, qm2 = 0, qm3 = 0, qn0 = 0, qn1 = 0, qn2 = 0, qn3 = 0, nset = 0;
+    int cbase0 = 0, cbase1 = 0;                         // CONV: tap-(0,0) offset, in-image taps
+    unsigned long long cmask0 = 0, cmask1 = 0;
+    int kh = 0, kw = 0, icc = 0;                        // CONV: tap, channel offset of the chunk
+    auto set_tap = [&]() {
+        const int to = (kh * cv.W + kw) * cv.Cin * 4;
+        const unsigned long long bit = 1ull << (kh * 8 + kw);
+        va0 = cmask0 & bit ? (unsigned)(cbase0 + to) : kOOB;
+        va1 = cmask1 & bit ? (unsigned)(cbase1 + to) : kOOB;
+    };
+    auto pixel = [&](int m, int& base, unsigned long long& mask) {
+        base = 0;
+        mask = 0;
+        if (m < M) {
+            const int hw = cv.OH * cv.OW;
+            const int n = m / hw, rem = m - n * hw;
+            const int oh = rem / cv.OW, ow = rem - oh * cv.OW;
+            const int ih0 = oh * cv.stride - cv.pad, iw0 = ow * cv.stride - cv.pad;
+            base = ((n * cv.H + ih0) * cv.W + iw0) * cv.Cin * 4 + 16 * aq;
+            unsigned rm = 0, cm = 0;
+            for (int d = 0; d < 8; ++d) {
+                rm |= ((unsigned)(ih0 + d) < (unsigned)cv.H) ? (1u << d) : 0u;
+                cm |= ((unsigned)(iw0 + d) < (unsigned)cv.W) ? (1u << d) : 0u;
+            }
+            for (int d = 0; d < 8; ++d)
+                if ((rm >> d) & 1u) mask |= (unsigned long long)cm << (8 * d);
+        }
+    };
     auto setup = [&](int k) {
         int m0, n0;
         tile_of(k, m0, n0);
-        in0 = n0;
-#pragma unroll
-        for (int t = 0; t < AIT; ++t) {
-            const int m = m0 + arow + 32 * t;
-            if (!CONV) {
-                arowoff[t] = m < M ? (unsigned)(m * lda + 4 * aq) * 4u : kOOB;
-            } else {
-                cbase[t] = 0;
-                cmask[t] = 0;
-                if (m < M) {
-                    const int hw = cv.OH * cv.OW;
-                    const int n = m / hw, rem = m - n * hw;
-                    const int oh = rem / cv.OW, ow = rem - oh * cv.OW;
-                    const int ih0 = oh * cv.stride - cv.pad, iw0 = ow * cv.stride - cv.pad;
-                    cbase[t] = ((n * cv.H + ih0) * cv.W + iw0) * cv.Cin * 4 + 16 * aq;
-                    unsigned rm = 0, cm = 0;
-                    for (int d = 0; d < 8; ++d) {
-                        rm |= ((unsigned)(ih0 + d) < (unsigned)cv.H) ? (1u << d) : 0u;
-                        cm |= ((unsigned)(iw0 + d) < (unsigned)cv.W) ? (1u << d) : 0u;
-                    }
-                    unsigned long long mk = 0;
-                    for (int d = 0; d < 8; ++d)
-                        if ((rm >> d) & 1u) mk |= (unsigned long long)cm << (8 * d);
-                    cmask[t] = mk;
-                }
-            }
-        }
-    };
-    // item t of the issue cursor's chunk into stage st (out of range when !live)
-    auto issue = [&](int t, float* st, bool live) {
-        const int k0 = ic * KC;
-        if (t < AIT) {
-            unsigned v = kOOB;
-            if (live) {
-                if (CONV) {
-                    const int tap = k0 / cv.Cin, ic0 = k0 - tap * cv.Cin;
-                    const int kh = tap / cv.KW, kw = tap - kh * cv.KW;
-                    if ((cmask[t] >> (kh * 8 + kw)) & 1ull)
-                        v = (unsigned)(cbase[t] + ((kh * cv.W + kw) * cv.Cin + ic0) * 4);
-                } else if (arowoff[t] != kOOB && !(kragged && k0 + 4 * aq >= K)) {
-                    v = arowoff[t] + (unsigned)k0 * 4u;
-                }
-            }
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, (lds_void32*)(st + (wave + 4 * t) * 256), 16, v, 0,
-                                                     0, 0);
+        qm3 = qm2; qm2 = qm1; qm1 = qm0; qm0 = m0;
+        qn3 = qn2; qn2 = qn1; qn1 = qn0; qn0 = n0;
+        ++nset;
+        sa = sb = 0;
+        // kOOB + n0 * 4 (or m0 * lda * 4) stays out of range
+        vb0 = n0 + bq4[0] < N ? brel0 + (unsigned)n0 * 4u : kOOB;
+        vb1 = n0 + bq4[1] < N ? brel1 + (unsigned)n0 * 4u : kOOB;
+        if (CONV) {
+            pixel(m0 + arow, cbase0, cmask0);
+            pixel(m0 + arow + 32, cbase1, cmask1);
+            kh = kw = icc = 0;
+            set_tap();
         } else {
-            const int tt = t - AIT;
-            const unsigned v = live && in0 + bq4[tt] < N && k0 + bkr[tt] < K
-                                   ? (unsigned)((k0 + bkr[tt]) * ldb + in0 + bq4[tt]) * 4u
-                                   : kOOB;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(bres, (lds_void32*)(st + SB + (wave + 4 * tt) * 256), 16, v,
-                                                     0, 0, 0);
+            va0 = m0 + arow < M ? arel + (unsigned)(m0 * lda) * 4u : kOOB;
+            va1 = m0 + arow + 32 < M ? arel + (unsigned)((m0 + 32) * lda) * 4u : kOOB;
         }
     };
-    auto advance = [&]() {
+    // the issue cursor's chunk into stage st
+    auto issue = [&](float* st) {
+        dma16(ares, st + wave * 256, va0, sa);
+        dma16(ares, st + (wave + 4) * 256, va1, sa);
+        dma16(bres, st + SB + wave * 256, vb0, sb);
+        dma16(bres, st + SB + (wave + 4) * 256, vb1, sb);
+    };
+    auto advance = [&]() {                              // the cursor to the next chunk
+        if (ik >= cnt) return;
         if (++ic == nch) {
             ic = 0;
-            if (++ik < cnt) setup(ik);
+            if (++ik < cnt) {
+                setup(ik);
+            } else {
+                sa = sb = 0;
+                va0 = va1 = vb0 = vb1 = kOOB;
+            }
+            return;
+        }
+        sb += (unsigned)(KC * 4) * ldb;
+        sa += KC * 4;
+        if (CONV) {                                     // a chunk lies in one tap (Cin % 64 == 0)
+            if ((icc += KC) == cv.Cin) {
+                icc = 0;
+                sa = 0;
+                if (++kw == cv.KW) { kw = 0; ++kh; }
+                set_tap();
+            }
+        } else if (kragged && ic == nch - 1) {          // the last chunk's k past K read zeros
+            va0 = ic * KC + 4 * aq < K ? va0 : kOOB;
+            va1 = ic * KC + 4 * aq < K ? va1 : kOOB;
+            vb0 = ic * KC + bkr[0] < K ? vb0 : kOOB;
+            vb1 = ic * KC + bkr[1] < K ? vb1 : kOOB;
         }
     };
 
@@ -587,22 +640,81 @@ __global__ __launch_bounds__(256) void k_gemm32p(const float* __restrict__ A,
     setup(0);
 #pragma unroll
     for (int a = 0; a < AHEAD; ++a) {
-        const bool live = a < nit;
-#pragma unroll
-        for (int t = 0; t < ITEMS; ++t) issue(t, sm + a * STAGE, live);
-        if (live) advance();
+        issue(sm + a * STAGE);
+        advance();
     }
 
+    // A finished tile's sums wait in fin[] and are stored during the next
+    // chunk, behind that chunk's DMA (flush): lane l, register e <-> row
+    // 32 wm + 8 (e / 4) + 4 h + e % 4, column 32 wn + r of the tile.  16 buffer
+    // stores of 128-byte row segments; columns past N carry kOOB.  A whole
+    // tile's row offsets are scalar (no address VALU); a tile that ends past
+    // M has them in the lane offset, which the range check surely covers.
+    f16v fin;
+    int fm0 = 0, fn0 = 0;
+    auto rows_of = [&](const float* p, int ldp) {       // the tile's rows of C or res as a buffer
+        const long long left = (long long)(M - fm0) * ldp * 4;
+        return __builtin_amdgcn_make_buffer_rsrc((void*)(p + (long long)fm0 * ldp), (short)0,
+                                                 (int)(left < 0x7fffffff ? left : 0x7fffffff), 0x00020000);
+    };
+    auto flush_rows = [&](auto whole) {
+        constexpr bool W = decltype(whole)::value;
+        const int rl = 32 * wm + 4 * h, cl = fn0 + 32 * wn + r;
+        const float fb = bias && cl < N ? bias[cl] : 0.f;
+        auto re = [](int e, int ldp) { return (unsigned)((8 * (e >> 2) + (e & 3)) * ldp) * 4u; };
+        if (res) {
+            const __amdgpu_buffer_rsrc_t rres = rows_of(res, ldr);
+            const unsigned ro = cl < N ? (unsigned)(rl * ldr + cl) * 4u : kOOB;
+#pragma unroll
+            for (int half = 0; half < 16; half += 8) {  // 8 rows at a time: 128 registers in all
+                float rv[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    rv[e] = __builtin_bit_cast(
+                        float, __builtin_amdgcn_raw_buffer_load_b32(rres, ro + (W ? 0u : re(half + e, ldr)),
+                                                                    W ? re(half + e, ldr) : 0u, 0));
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    float v = fin[half + e];
+                    if (bias) v = v + fb;
+                    fin[half + e] = v + rv[e];
+                }
+                asm volatile("" ::: "memory");
+            }
+        } else if (bias) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) fin[e] = fin[e] + fb;
+        }
+        if (act == 1) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) fin[e] = act_apply(fin[e], 1);
+        } else if (act == 2) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) fin[e] = act_apply(fin[e], 2);
+        }
+        const __amdgpu_buffer_rsrc_t cres = rows_of(C, ldc);
+        const unsigned co = cl < N ? (unsigned)(rl * ldc + cl) * 4u : kOOB;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)                    // 16 = sc1: written through L2
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(fin[e]), cres,
+                                                  co + (W ? 0u : re(e, ldc)), W ? re(e, ldc) : 0u, 16);
+    };
+    auto flush = [&]() {
+        if (fm0 + BM <= M) flush_rows(std::true_type{});
+        else flush_rows(std::false_type{});
+    };
+
     int st = 0, ck = 0, cc = 0;
+    bool pend = false, stored = false;
     for (int g = 0; g < nit; ++g) {
-        // Chunk g has landed once at most the (AHEAD - 1) * ITEMS loads issued
-        // after it are outstanding: loads complete in issue order, and the
-        // epilogue's inline-asm stores queued among them only lengthen the wait.
-        __builtin_amdgcn_s_waitcnt(g32_vmcnt((AHEAD - 1) * ITEMS));
+        // Chunk g has landed once at most the loads and stores issued after
+        // its DMA are outstanding (vmcnt counts them in issue order): the
+        // (AHEAD - 1) * ITEMS loads of later chunks, and a flush's 16 stores.
+        if (stored) __builtin_amdgcn_s_waitcnt(g32_vmcnt((AHEAD - 1) * ITEMS + 16));
+        else __builtin_amdgcn_s_waitcnt(g32_vmcnt((AHEAD - 1) * ITEMS));
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         const float* S = sm + st * STAGE;
         float* NA = sm + (st == 0 ? NST - 1 : st - 1) * STAGE;   // (g + AHEAD) % NST
-        const bool more = g + AHEAD < nit;
         f4g a[AQ];
         float bb[KSTEP];
 #pragma unroll
@@ -612,73 +724,26 @@ __global__ __launch_bounds__(256) void k_gemm32p(const float* __restrict__ A,
 #pragma unroll
         for (int k = 0; k < KSTEP; ++k) {
             acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[k >> 2][k & 3], bb[k], acc, 0, 0, 0);
-            if (k == 1) {
-#pragma unroll
-                for (int t = 0; t < ITEMS; ++t) issue(t, NA, more);
-            }
+            if (k == 1) issue(NA);
         }
-        if (more) advance();
+        asm volatile("" ::: "memory");                  // the stores stay behind the DMA
+        advance();
+        if (pend) flush();
+        stored = pend;
+        pend = false;
         st = st == NST - 1 ? 0 : st + 1;
         if (++cc < nch) continue;
         cc = 0;
-        // ---- epilogue of tile ck through the stage of its last chunk
-        int m0, n0;
-        tile_of(ck, m0, n0);
+        const int back = nset - 1 - ck;                  // setups since this tile's
+        fm0 = back == 0 ? qm0 : back == 1 ? qm1 : back == 2 ? qm2 : qm3;
+        fn0 = back == 0 ? qn0 : back == 1 ? qn1 : back == 2 ? qn2 : qn3;
         ++ck;
-        float* const stg = sm + (st == 0 ? NST - 1 : st - 1) * STAGE;
-        auto sidx = [](int rr, int cq) { return rr * 64 + ((((cq >> 2) ^ (((rr >> 2) & 1) << 3))) << 2) + (cq & 3); };
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        fin = acc;
+        pend = true;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int rr = 32 * wm + 8 * (e >> 2) + 4 * h + (e & 3);
-            stg[sidx(rr, col)] = acc[e];
-            acc[e] = 0.f;
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        const int q = tid & 15, n = n0 + 4 * q;
-        f4g bq = {0.f, 0.f, 0.f, 0.f};
-        if (bias) {
-            if (vec && n + 4 <= N) {
-                bq = *(const f4g*)(bias + n);
-            } else {
-#pragma unroll
-                for (int kq = 0; kq < 4; ++kq) bq[kq] = n + kq < N ? bias[n + kq] : 0.f;
-            }
-        }
-        const bool full = m0 + BM <= M && n0 + BN <= N;
-        f4g rv[4];
-        if (res && vec && full) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                rv[i] = *(const f4g*)(res + (long long)(m0 + (tid >> 4) + 16 * i) * ldr + n);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int rr = (tid >> 4) + 16 * i, m = m0 + rr;
-            if (m >= M) continue;
-            f4g v = *(const f4g*)&stg[sidx(rr, 4 * q)];
-            float* dst = C + (long long)m * ldc + n;
-            if (vec && n + 4 <= N) {
-                if (bias) v = v + bq;
-                if (res) v = v + (full ? rv[i] : *(const f4g*)(res + (long long)m * ldr + n));
-#pragma unroll
-                for (int kq = 0; kq < 4; ++kq) v[kq] = act_apply(v[kq], act);
-                // s_nop: a VALU write to the data registers of a store of more
-                // than 8 bytes needs a wait state after it
-                asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(dst), "v"(v) : "memory");
-            } else {
-#pragma unroll
-                for (int kq = 0; kq < 4; ++kq) {
-                    if (n + kq >= N) continue;
-                    float w = v[kq];
-                    if (bias) w = w + bq[kq];
-                    if (res) w = w + res[(long long)m * ldr + n + kq];
-                    w = act_apply(w, act);
-                    asm volatile("global_store_dword %0, %1, off sc1" ::"v"(dst + kq), "v"(w) : "memory");
-                }
-            }
-        }
+        for (int e = 0; e < 16; ++e) acc[e] = 0.f;
     }
+    flush();
     __builtin_amdgcn_s_waitcnt(g32_vmcnt(0));          // the out-of-range loads and the stores
 }
 
@@ -692,7 +757,7 @@ struct G32Tile { int bm, bn, nst, ks = 1, kc = 64, pers = 0; };
 // tiles at every K, since one workgroup per CU leaves the DMA latency and the
 // epilogue exposed.  ACFUN_G32_KMIN=<K> enables the larger tiles from that K
 // (sweeps).  Three stages when the 64 x 64 grid is a single wave of workgroups.
-G32Tile pick_g32(int M, int N, int K) {
+G32Tile pick_g32(int M, int N, int K, bool conv) {
     const long long cus = num_cus();
     const int nch = (K + 63) / 64;
     auto tiles = [&](int bm, int bn) {
@@ -709,14 +774,18 @@ G32Tile pick_g32(int M, int N, int K) {
     // workgroup split K (two waves per SIMD instead of one).
     static const bool ks_off = getenv("ACFUN_G32_NOKS") != nullptr;
     if (!ks_off && nch >= 8 && tiles(64, 64) <= cus) return G32Tile{64, 64, 2, 2};
-    // Two or more 64 x 64 tiles per CU: the persistent kernel, two stages,
-    // four workgroups per CU (config 5, fp32: 5.71 -> 5.09 ms per batch of 64;
-    // three stages at three per CU: 5.33 ms).  ACFUN_G32P=0 turns it off.
+    // More 64 x 64 tiles than CUs: the persistent kernel, two stages, four
+    // workgroups per CU.  A GEMM from one tile per CU on (3136 x 512 tiles, 392:
+    // K = 64, 256, 512, 2048 take 5.7, 11.6, 19.9, 66.9 us, one tile per
+    // workgroup 7.8, 14.7, 23.4, 73.4); a convolution from two (3x3/2 over
+    // 14 x 14 x 512, batch 64, 392 tiles: 166 against 160 us -- a tile's pixel
+    // set-up is not hidden when most workgroups run a single tile).
+    // ACFUN_G32P=0 turns it off.
     static const bool pers = [] {
         const char* e = getenv("ACFUN_G32P");
         return !(e && atoi(e) == 0);
     }();
-    if (pers && tiles(64, 64) >= 2 * cus) return G32Tile{64, 64, 2, 1, 32, 1};
+    if (pers && (conv ? tiles(64, 64) >= 2 * cus : tiles(64, 64) > cus)) return G32Tile{64, 64, 2, 1, 32, 1};
     // Three stages (one workgroup per CU) only when the tiles fit in one wave;
     // between one and two tiles per CU two stages at two workgroups per CU
     // (config 5's 392-tile layers: GEMM 3136 x 512 x 2048 94.9 -> 81.0 us,
@@ -769,11 +838,9 @@ bool launch_g32p(int M, int N, int K, const float* A, int lda, const float* B, i
     const long long tiles = (long long)((M + 63) / 64) * ((N + 63) / 64);
     const long long slots = (NST == 2 ? 4ll : 3ll) * num_cus(), need = (tiles + 7) / 8 * 8;
     const unsigned grid = (unsigned)(slots < need ? slots : need);
-    auto al = [](const void* q) { return ((uintptr_t)q & 15u) == 0; };
-    const int vec = al(C) && ldc % 4 == 0 && (!bias || al(bias)) && (!res || (al(res) && ldr % 4 == 0));
     const unsigned a_bytes = CONV ? cv.bytes : (unsigned)((long long)M * lda * 4);
     ACFUN_LAUNCH("k_gemm32", (k_gemm32p<NST, CONV>), dim3(grid), dim3(256), lds, s, A, B, C, bias, res, M, N,
-                 K, lda, ldb, ldc, ldr, act, vec, a_bytes, cv);
+                 K, lda, ldb, ldc, ldr, act, a_bytes, cv);
     return check_launch("k_gemm32p");
 }
 
@@ -796,10 +863,11 @@ int g32_index(const G32Tile& t) {
     return 0;
 }
 // K groups need chunks for every group: at least two each.
-// The persistent kernel addresses A through one 32-bit buffer resource.
-bool g32_admits(int c, int K, long long a_bytes) {
+// The persistent kernel addresses A through one 32-bit buffer resource,
+// and a tile's rows of C and of the residual through others.
+bool g32_admits(int c, int K, long long a_bytes, int ldc, int ldr) {
     const G32Tile& t = kG32Cand[c];
-    if (t.pers) return a_bytes < 0x7fffffffll;
+    if (t.pers) return a_bytes < 0x7fffffffll && 64ll * (ldc > ldr ? ldc : ldr) * 4 < 0x7fffffffll;
     return t.ks == 1 || (K + t.kc - 1) / t.kc >= 2 * t.ks;
 }
 
@@ -839,8 +907,8 @@ TuneMaker g32_maker(int M, int N, int K, const G32Conv& cv) {
             hipMemsetD32Async((hipDeviceptr_t)b->p, kTuneFill, bbytes / 4, s) != hipSuccess)
             return TuneRunner();
         return [=](int cand, hipStream_t st) {
-            if (cand < 0) cand = g32_index(pick_g32(M, N, K));     // the built-in choice
-            if (!g32_admits(cand, K, CONV ? (long long)cv.bytes : (long long)M * K * 4)) return false;
+            if (cand < 0) cand = g32_index(pick_g32(M, N, K, CONV));     // the built-in choice
+            if (!g32_admits(cand, K, CONV ? (long long)cv.bytes : (long long)M * K * 4, N, 0)) return false;
             return launch_cand<CONV>(cand, M, N, K, a->as<float>(), CONV ? cv.Cin : K, b->as<float>(), N,
                                      c->as<float>(), N, nullptr, 0, st, nullptr, 0, cv);
         };
@@ -865,8 +933,8 @@ bool launch_gemm32(int M, int N, int K, const float* A, int lda, const float* B,
         }
     }
     const long long a_bytes = CONV ? (long long)cv.bytes : (long long)M * lda * 4;
-    if (c < 0 || !g32_admits(c, K, a_bytes)) c = g32_index(pick_g32(M, N, K));
-    if (!g32_admits(c, K, a_bytes)) c = 0;
+    if (c < 0 || !g32_admits(c, K, a_bytes, ldc, ldr)) c = g32_index(pick_g32(M, N, K, CONV));
+    if (!g32_admits(c, K, a_bytes, ldc, ldr)) c = 0;
     return launch_cand<CONV>(c, M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
 }
 }  // namespace
