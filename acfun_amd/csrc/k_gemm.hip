@@ -342,7 +342,19 @@ bool aligned16(const void* q) { return ((uintptr_t)q & 15u) == 0; }
 template <bool CONV>
 bool run(GemmP p, int batch, bool va, bool vb, hipStream_t s, const TileCfg* force = nullptr) {
     if (p.M <= 0 || p.N <= 0) return true;
-    TileCfg c = force ? *force : tuned_f32_tile(p.M, p.N, p.K, batch);
+    bool searched = force != nullptr;
+    TileCfg c = force ? *force : tuned_f32_tile(p.M, p.N, p.K, batch, &searched);
+    // k_gemms's tiles, which take any alignment, unless the search chose a tile
+    const GsAlt alt = c.split > 1 ? GsAlt::SPLITK : GsAlt::F32;
+    if (!searched && batch == 1 && p.K > 0) {
+        if (CONV) {
+            const ConvShape g{p.M / (p.OH * p.OW), p.H, p.W, p.Cin, p.K / (p.KW * p.Cin), p.KW,
+                              p.stride, p.pad, p.OH, p.OW};
+            if (convs_wins(g, p.N, alt)) return convs_f32(g, p.A, p.B, p.bias, p.N, p.C, p.act, s);
+        } else if (gemms_wins(p.M, p.N, p.K, p.lda, p.ldb, alt)) {
+            return gemms_f32(p.M, p.N, p.K, p.A, p.lda, p.B, p.ldb, p.C, p.ldc, p.bias, p.act, s);
+        }
+    }
     if (batch > 1) c.split = 1;
     int splits = c.split < 1 ? 1 : c.split;
     int kchunk = (p.K + splits - 1) / splits;
@@ -406,7 +418,7 @@ TileCfg f32_cand(int c) {
     return TileCfg{tiles[c / 4][0], tiles[c / 4][1], splits[c % 4]};
 }
 
-TileCfg tuned_f32_tile(int M, int N, int K, int batch) {
+TileCfg tuned_f32_tile(int M, int N, int K, int batch, bool* searched) {
     const TileCfg d = default_f32_tile(M, N, K, batch);
     if (batch != 1) return d;
     const std::vector<int> key{M, N, K};
@@ -425,10 +437,14 @@ TileCfg tuned_f32_tile(int M, int N, int K, int batch) {
                 return TuneRunner();
             return [=](int cand, hipStream_t st) {
                 const TileCfg t = cand < 0 ? default_f32_tile(M, N, K) : f32_cand(cand);
+                if (cand < 0 && gemms_wins(M, N, K, K, N, t.split > 1 ? GsAlt::SPLITK : GsAlt::F32))
+                    return gemms_f32(M, N, K, a->as<float>(), K, b->as<float>(), N, cc->as<float>(), N, nullptr,
+                                     0, st);
                 if (t.split > 1 && K < 256 * t.split) return false;
                 return gemm_f32_cfg(M, N, K, a->as<float>(), b->as<float>(), cc->as<float>(), t, st);
             };
         });
+    if (searched) *searched = c >= 0;
     return c >= 0 ? f32_cand(c) : d;
 }
 
@@ -442,9 +458,10 @@ bool gemm_f32(int M, int N, int K, const float* A, int lda, const float* B, int 
     if (K <= 0) {  // empty reduction: C = bias / 0 (then ReLU), like the reference loops
         p.K = 0;
     }
-    // Few output tiles and a long K (an FC layer): the split-K register-staged
-    // kernel spreads K over the CUs that k_gemm32's tiles leave idle (batch-64
-    // FC 2048 -> 1000: 40.8 -> 16.7 us; 4096 -> 4096: 76 -> 44 us).
+    // Few output tiles and a long K (an FC layer) belong to the split-K
+    // family: k_gemms's tiles up to K of some 6,000, past that the register-
+    // staged kernel with K spread over the idle CUs (batch-64 FC 2048 -> 1000:
+    // 7.4 us; one tile per CU takes 40.8, split-K with its reduce launch 17.4).
     // ACFUN_FC_SPLITK=0 turns it off.
     static const bool fcs = [] {
         const char* e = getenv("ACFUN_FC_SPLITK");

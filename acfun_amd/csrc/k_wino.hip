@@ -1551,6 +1551,8 @@ bool w23_default(const float* in, const float* Up, const float* bias, float* out
 TuneMaker w23_maker(int N, int H, int W, int Cin, int Cout) {
     return [=]() -> TuneRunner {
         const int Cinp = (Cin + 15) / 16 * 16, tH = (H + 1) / 2, tW = (W + 1) / 2;
+        const ConvShape g{N, H, W, Cin, 3, 3, 1, 1, H, W};
+        // ub also holds the 9 Cin x Cout weights of the direct convolution
         const size_t ib = (size_t)N * H * W * Cin * 4, ub = (size_t)16 * Cout * Cinp * 4,
                      ob = (size_t)N * H * W * Cout * 4;
         if (ib + ub + ob > ((size_t)2 << 30)) return TuneRunner();
@@ -1562,6 +1564,8 @@ TuneMaker w23_maker(int N, int H, int W, int Cin, int Cout) {
             hipMemsetD32Async((hipDeviceptr_t)u->p, kTuneFill, ub / 4, s) != hipSuccess)
             return TuneRunner();
         return [=](int cand, hipStream_t st) {
+            if (cand < 0 && convs_wins(g, Cout, GsAlt::WINO))
+                return convs_f32(g, x->as<float>(), u->as<float>(), nullptr, Cout, o->as<float>(), 0, st);
             if (cand < 0)
                 return w23_default(x->as<float>(), u->as<float>(), nullptr, o->as<float>(), N, H, W, Cin,
                                    Cinp, Cout, tH, tW, 0, st);
@@ -1575,9 +1579,10 @@ TuneMaker w23_maker(int N, int H, int W, int Cin, int Cout) {
 }
 
 // Upre: the filter already transformed for this shape's plan (a model's cached
-// transform), or null to transform it here.
+// transform), or null to transform it here.  direct: a shape with few output
+// tiles may run as a direct convolution (k_gemms.hip).
 bool run_wino23(const float* in, int N, int H, int W, int Cin, const float* w, const float* bias,
-                int Cout, float* out, int act, hipStream_t s, const float* Upre = nullptr) {
+                int Cout, float* out, int act, hipStream_t s, const float* Upre, bool direct) {
     int tH = (H + 1) / 2, tW = (W + 1) / 2;
     int Cinp = (Cin + 15) / 16 * 16;
     const int plan = wino23_plan_impl(N, H, W, Cin, Cout, in);
@@ -1585,16 +1590,23 @@ bool run_wino23(const float* in, int N, int H, int W, int Cin, const float* w, c
         ConvShape gs{N, H, W, Cin, 3, 3, 1, 1, H, W};
         return conv_igemm_f32(gs, in, w, bias, Cout, out, act, s);
     }
+    // the tile search's choice of unit kernel for this shape, if any
+    int c = -1;
+    if (plan == 1) {
+        const std::vector<int> key{N, H, W, Cin, Cout};
+        bool rec = false;
+        c = tune_lookup("w23", key, kW23NC, &rec);
+        if (rec) tune_record("w23", key, kW23NC, w23_maker(N, H, W, Cin, Cout));
+    }
+    // the conv routes may multiply few output tiles directly instead
+    const ConvShape gd{N, H, W, Cin, 3, 3, 1, 1, H, W};
+    if (direct && c < 0 && convs_wins(gd, Cout, GsAlt::WINO))
+        return convs_f32(gd, in, w, bias, Cout, out, act, s);
     Scratch Uown(Upre ? 0 : (size_t)16 * Cout * Cinp * sizeof(float), s);
     if (!Upre && !Uown.p) return false;
     const float* Up = Upre ? Upre : Uown.as<float>();
     if (plan == 1) {
         if (!Upre && !wino23_filter_impl(w, Cin, Cout, 1, Uown.as<float>(), s)) return false;
-        // the tile search's choice of unit kernel for this shape, if any
-        const std::vector<int> key{N, H, W, Cin, Cout};
-        bool rec = false;
-        const int c = tune_lookup("w23", key, kW23NC, &rec);
-        if (rec) tune_record("w23", key, kW23NC, w23_maker(N, H, W, Cin, Cout));
         if (c >= 0) {
             bool launched = false;
             if (!w23_launch(c, in, Up, bias, out, N, H, W, Cin, Cinp, Cout, tH, tW, act, s, &launched))
@@ -1687,7 +1699,12 @@ bool winograd_f32(int tile, const float* in, int N, int H, int W, int Cin, const
         if (done) return true;
         return run_fused<4, 16, 4, 8>(in, N, H, W, Cin, w, bias, Cout, out, act, s);
     }
-    return run_wino23(in, N, H, W, Cin, w, bias, Cout, out, act, s, Upre);
+    return run_wino23(in, N, H, W, Cin, w, bias, Cout, out, act, s, Upre, false);
+}
+
+bool wino23_direct(int N, int H, int W, int Cin, int Cout) {
+    const ConvShape g{N, H, W, Cin, 3, 3, 1, 1, H, W};
+    return convs_wins(g, Cout, GsAlt::WINO) && !tune_has("w23", std::vector<int>{N, H, W, Cin, Cout}, kW23NC);
 }
 
 bool winograd_route_f32(int tile, const float* in, int N, int H, int W, int Cin, const float* w,
@@ -1710,7 +1727,9 @@ bool winograd_route_f32(int tile, const float* in, int N, int H, int W, int Cin,
     // 7 x 7 stage, run units of two images' tile blocks.)
     ConvShape g{N, H, W, Cin, 3, 3, 1, 1, H, W};
     if (!unit23 && conv32_ok(g, Cout, in, w)) return conv32_f32(g, in, w, bias, Cout, out, act, s);
-    return winograd_f32(tile, in, N, H, W, Cin, w, bias, Cout, out, act, s, tile == 2 ? Upre : nullptr);
+    if (tile == 2 && N > 0 && H > 0 && W > 0)
+        return run_wino23(in, N, H, W, Cin, w, bias, Cout, out, act, s, Upre, true);
+    return winograd_f32(tile, in, N, H, W, Cin, w, bias, Cout, out, act, s, nullptr);
 }
 
 }  // namespace acfun

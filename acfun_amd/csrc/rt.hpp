@@ -193,6 +193,18 @@ bool gemm32_f32(int M, int N, int K, const float* A, int lda, const float* B, in
 bool conv32_ok(const ConvShape& g, int Cout, const float* in, const float* w);
 bool conv32_f32(const ConvShape& g, const float* in, const float* w, const float* bias, int Cout,
                 float* out, int act, hipStream_t s, const float* res = nullptr, int ldr = 0);
+// Few output tiles, or operands of any alignment (k_gemms.hip): small tiles
+// whose K range a workgroup's waves split.  gemms_wins / convs_wins say whether
+// the shape is admitted (a convolution: Cin a multiple of 16, KH and KW <= 8)
+// and this is the faster kernel than `alt`, the one it would otherwise run.
+enum class GsAlt { G32, CONV32, F32, SPLITK, WINO };
+bool gemms_wins(int M, int N, int K, int lda, int ldb, GsAlt alt);
+bool gemms_f32(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
+               int ldc, const float* bias, int act, hipStream_t s, const float* res = nullptr,
+               int ldr = 0);
+bool convs_wins(const ConvShape& g, int Cout, GsAlt alt);
+bool convs_f32(const ConvShape& g, const float* in, const float* w, const float* bias, int Cout,
+               float* out, int act, hipStream_t s, const float* res = nullptr, int ldr = 0);
 bool gemm_f32(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
               int ldc, const float* bias, int act, hipStream_t s);
 bool conv_igemm_f32(const ConvShape& g, const float* in, const float* w, const float* bias,
@@ -244,6 +256,9 @@ bool run_wino43(const float* in, int N, int H, int W, int Cin, const float* w, c
 // would use; both tiles compute the direct convolution exactly over the
 // rationals, so the faster kernel for the shape runs (within the Winograd
 // tolerance of the reference either way).
+// wino23_direct: a 3x3/s1/p1 shape that winograd_route_f32 multiplies directly
+// (few output tiles, no searched choice of unit kernel): no filter transform.
+bool wino23_direct(int N, int H, int W, int Cin, int Cout);
 bool winograd_route_f32(int tile, const float* in, int N, int H, int W, int Cin, const float* w,
                         const float* bias, int Cout, float* out, int act, hipStream_t s,
                         const float* Upre = nullptr);
@@ -402,6 +417,7 @@ using TuneRunner = std::function<bool(int cand, hipStream_t s)>;
 using TuneMaker = std::function<TuneRunner()>;
 const char* device_arch();      // the current device's gfx name, e.g. "gfx950"
 int tune_lookup(const char* kind, const std::vector<int>& key, int ncand, bool* record);
+bool tune_has(const char* kind, const std::vector<int>& key, int ncand);   // a searched candidate exists
 void tune_record(const char* kind, const std::vector<int>& key, int ncand, TuneMaker maker);
 bool autotune_wanted();         // ACFUN_AUTOTUNE=1: true at the first ask of a process
 // The replays fill their fp32 operands with this bit pattern (0.01f), not
@@ -414,7 +430,7 @@ const char* tune_status();
 // k_gemm_f32 tiles (the unaligned fallback).
 struct TileCfg { int bm, bn, split; };
 TileCfg default_f32_tile(int M, int N, int K, int batch = 1);
-TileCfg tuned_f32_tile(int M, int N, int K, int batch = 1);
+TileCfg tuned_f32_tile(int M, int N, int K, int batch = 1, bool* searched = nullptr);
 // Runs one fp32 GEMM with an explicit tile config (used by the tile search).
 bool gemm_f32_cfg(int M, int N, int K, const float* A, const float* B, float* C,
                   const TileCfg& cfg, hipStream_t s);

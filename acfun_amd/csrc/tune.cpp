@@ -151,6 +151,14 @@ int tune_lookup(const char* kind, const std::vector<int>& key, int ncand, bool* 
     return -1;
 }
 
+bool tune_has(const char* kind, const std::vector<int>& key, int ncand) {
+    const TKey k{device_arch(), kind, key};
+    std::lock_guard<std::mutex> lk(g_mu);
+    load_cache_locked();
+    auto it = g_table.find(k);
+    return it != g_table.end() && it->second.second == ncand && it->second.first >= 0;
+}
+
 void tune_record(const char* kind, const std::vector<int>& key, int ncand, TuneMaker maker) {
     TKey k{device_arch(), kind, key};
     std::lock_guard<std::mutex> lk(g_mu);
