@@ -8,13 +8,27 @@
 //
 // One packing launch writes the rounded operands k-contiguous -- A as
 // [M][Kp], B transposed as [N][Kp], Kp = K rounded up to 128, zeros beyond K
-// -- and k_bf16mm multiplies them on v_mfma_f32_32x32x16_bf16: 64 x 64 tiles,
-// 2 x 2 waves, K in chunks of 256 bytes (128 bf16) DMA'd into LDS by
-// buffer_load_dwordx4 ... lds, quad q of row r at slot r*16 + (q ^ (r % 16)),
-// four stages (three chunks ahead).  In k-step s lane half h reads quad 2s+h
-// of its A row and its B row: eight bf16 each, the MFMA's 16 k per step.  At
-// 1024^3 the grid is one tile per CU and the K loop is bound by the DMA round
-// trip, so the chunks are large and many are in flight.
+// -- and k_bf16mm multiplies them on v_mfma_f32_32x32x16_bf16.
+//
+// k_bf16mm: WM x WN waves, each FM x FN accumulators of 32 x 32; K in chunks
+// of KB bytes DMA'd into LDS by buffer_load_dwordx4 ... lds (lane offsets fixed,
+// one scalar offset per chunk), NST stages.  In k-step s of a chunk lane half h
+// reads quad 2s + h of its A rows and B rows: eight bf16 each, the MFMA's 16 k.
+// A k-step's operands are read while the step before is multiplied, and the
+// last step's MFMAs cover the barrier and the first reads of the next chunk
+// (64 x 64 tiles, one MFMA per step, read the whole chunk up front).
+//
+// What bounds a large product is LDS: a wave of FM x FN blocks reads
+// 32 (FM + FN) bytes per lane pair for FM x FN MFMAs, and with 64 x 64 tiles (FM
+// = FN = 1) that and the DMA writes take four times the MFMA time.  256 x 256
+// tiles on eight 128 x 64 waves bring LDS down to about the MFMA time, at one
+// workgroup per CU; they need 256 tiles to fill the chip.  Measured, us for
+// k_bf16mm alone with 64 x 64 (every size's tile before) / 128 x 128 / 256 x 256:
+//   4096^3              289 / 127 / 111 (1,234 TFLOP/s)
+//   3008 x 2000 x 4096  109 /  54 /  81
+//   2048^3               41 /  21 /  44
+//   1024^3              6.9 / 11.9 / 25
+// With the packing launch (5.7 TB/s) 4096^3 takes 146 us, 325 before.
 #include "rt.hpp"
 
 namespace acfun {
@@ -111,113 +125,183 @@ __global__ __launch_bounds__(256) void k_pack_bf16(const float* __restrict__ A, 
     else pack_bt_bf16(b - nba, B, K, N, ldb, Bt, Kp, vb != 0);
 }
 
-constexpr int BF_BM = 64, BF_BN = 64, BF_NST = 4, BF_KB = 256;   // K chunk: 256 bytes, 128 bf16
-constexpr int BF_SA = BF_BM * BF_KB, BF_STG = (BF_BM + BF_BN) * BF_KB;
-static_assert(BF_NST == 4, "the waits below leave at most two chunks in flight");
 // s_waitcnt vmcnt(n), n < 64
 constexpr int bf_vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0F70; }
 
-__global__ __launch_bounds__(256) void k_bf16mm(const unsigned short* __restrict__ Ab,
-                                                const unsigned short* __restrict__ Bt,
-                                                float* __restrict__ C, int M, int N, int Kp,
-                                                int ldc, unsigned a_bytes, unsigned b_bytes) {
-    constexpr int AIT = BF_BM / 16, BIT = BF_BN / 16, ITEMS = AIT + BIT;   // 1 KB (4 rows) per item
-    constexpr int AHEAD = BF_NST - 1;
+__device__ __forceinline__ void bf_dma16(__amdgpu_buffer_rsrc_t rsrc, char* lds, unsigned voff, unsigned soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void*)lds, 16, voff, soff, 0, 0);
+}
+
+template <int WM, int WN, int FM, int FN, int KB, int NST>
+struct BfTile {
+    static constexpr int BM = 32 * WM * FM, BN = 32 * WN * FN, T = 64 * WM * WN;
+    static constexpr int SA = BM * KB, STG = (BM + BN) * KB, LDS = NST * STG;
+};
+
+template <int WM, int WN, int FM, int FN, int KB, int NST>
+__global__ __launch_bounds__(64 * WM * WN) void k_bf16mm(const unsigned short* __restrict__ Ab,
+                                                         const unsigned short* __restrict__ Bt,
+                                                         float* __restrict__ C, int M, int N, int Kp,
+                                                         int ldc, unsigned a_bytes, unsigned b_bytes) {
+    using Tl = BfTile<WM, WN, FM, FN, KB, NST>;
+    constexpr int BM = Tl::BM, BN = Tl::BN, NW = WM * WN;
+    constexpr int QR = KB / 16, RPI = 64 / QR;          // quads per row, rows per DMA instruction
+    constexpr int AIT = BM / RPI / NW, BIT = BN / RPI / NW, ITEMS = AIT + BIT;
+    constexpr int KS = KB / 32;                         // k-steps of 16 per chunk
     constexpr unsigned kOOB = 0x80000000u;
+    static_assert(AIT * RPI * NW == BM && BIT * RPI * NW == BN, "whole DMA instructions per wave");
+    static_assert(KS % 2 == 0 && NST >= 2 && (NST - 1) * ITEMS < 64, "operand sets, vmcnt");
     extern __shared__ __attribute__((aligned(16))) char smb[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
-    // XCD-contiguous tile order (workgroup id mod 8 = XCD)
-    const int gn = (N + BF_BN - 1) / BF_BN, total = gn * ((M + BF_BM - 1) / BF_BM);
-    int L = blockIdx.x;
-    if ((total & 7) == 0) L = (L & 7) * (total >> 3) + (L >> 3);
-    const int m0 = (L / gn) * BF_BM, n0 = (L % gn) * BF_BN;
-    const int nch = Kp >> 7;
+    const int wm = wave / WN, wn = wave - wm * WN;
+    // XCD x (workgroup id mod 8) owns a contiguous run of tiles; a run goes in
+    // groups of 4 tile rows, column-major inside, so the tiles an XCD runs
+    // together are a compact patch whose operands share its L2
+    const int gn = (N + BN - 1) / BN, gm = (M + BM - 1) / BM, total = gn * gm;
+    const int x = blockIdx.x & 7;
+    const int L = (int)(((long long)x * total) >> 3) + (int)(blockIdx.x >> 3);
+    if (L >= (int)(((long long)(x + 1) * total) >> 3)) return;
+    constexpr int GRP = 4;
+    const int grp = L / (GRP * gn), rows = gm - grp * GRP < GRP ? gm - grp * GRP : GRP;
+    const int rin = L - grp * GRP * gn;
+    const int m0 = (grp * GRP + rin % rows) * BM, n0 = (rin / rows) * BN;
+    const int nch = Kp / (KB / 2);
     const __amdgpu_buffer_rsrc_t ares =
         __builtin_amdgcn_make_buffer_rsrc((void*)Ab, (short)0, (int)a_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t bres =
         __builtin_amdgcn_make_buffer_rsrc((void*)Bt, (short)0, (int)b_bytes, 0x00020000);
-    // DMA rows of this lane: row 4*(wave + 4t) + lane/16, slot lane%16 holding
-    // quad (lane%16) ^ (row%16)
-    const int sl = lane & 15, rl = lane >> 4;
+    // quad q of row r sits at slot q ^ sw(r): 8 consecutive rows' reads of one
+    // quad cover all banks
+    auto sw = [](int r) { return QR >= 8 ? r & (QR - 1) : (r >> 1) & (QR - 1); };
+    const int sl = lane % QR, rl = lane / QR;
     unsigned av[AIT], bv[BIT];
 #pragma unroll
     for (int t = 0; t < AIT; ++t) {
-        const int row = 4 * (wave + 4 * t) + rl, q = sl ^ (row & 15);
+        const int row = RPI * (wave + NW * t) + rl, q = sl ^ sw(row);
         av[t] = m0 + row < M ? (unsigned)((m0 + row) * Kp * 2 + 16 * q) : kOOB;
     }
 #pragma unroll
     for (int t = 0; t < BIT; ++t) {
-        const int row = 4 * (wave + 4 * t) + rl, q = sl ^ (row & 15);
+        const int row = RPI * (wave + NW * t) + rl, q = sl ^ sw(row);
         bv[t] = n0 + row < N ? (unsigned)((n0 + row) * Kp * 2 + 16 * q) : kOOB;
     }
-    auto issue = [&](int t, int c, char* st) {
-        if (t < AIT) {
-            const unsigned v = av[t] + (unsigned)(c << 8);   // kOOB + k stays out of range
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, (lds_void*)(st + (wave + 4 * t) * 1024), 16,
-                                                     v, 0, 0, 0);
-        } else {
-            const int tt = t - AIT;
-            const unsigned v = bv[tt] + (unsigned)(c << 8);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(bres, (lds_void*)(st + BF_SA + (wave + 4 * tt) * 1024),
-                                                     16, v, 0, 0, 0);
-        }
+    // Every iteration issues one chunk (past the end the last one again, into a
+    // stage that is not read), so all waits of the loop are the same.
+    auto issue = [&](int c, char* st) {
+        const unsigned so = (unsigned)(c < nch ? c : nch - 1) * KB;
+#pragma unroll
+        for (int t = 0; t < AIT; ++t) bf_dma16(ares, st + (wave + NW * t) * 1024, av[t], so);
+#pragma unroll
+        for (int t = 0; t < BIT; ++t) bf_dma16(bres, st + Tl::SA + (wave + NW * t) * 1024, bv[t], so);
     };
-    // LDS read offsets (bytes within a stage) per k-step
+    // LDS read offsets of k-step s: a lane's quad 2 s + h of its rows
     const int r32 = lane & 31, hq = lane >> 5;
-    const int ra = wm * 32 + r32, rb = wn * 32 + r32;
-    int rda[8], rdb[8];
+    const int ra = wm * 32 * FM + r32, rb = wn * 32 * FN + r32;     // + 32 i: the same swizzle
+    int qo[KS];
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        rda[s] = ra * BF_KB + 16 * ((2 * s + hq) ^ (ra & 15));
-        rdb[s] = BF_SA + rb * BF_KB + 16 * ((2 * s + hq) ^ (rb & 15));
-    }
-    f16v acc;
+    for (int s = 0; s < KS; ++s) qo[s] = 16 * ((2 * s + hq) ^ sw(r32));
+    f16v acc[FM][FN];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
+    auto read = [&](i4v (&a)[FM], i4v (&b)[FN], const char* S, int s) {
 #pragma unroll
-    for (int a = 0; a < AHEAD; ++a)
-        if (a < nch) {
+        for (int i = 0; i < FM; ++i) a[i] = *(const i4v*)(S + (ra + 32 * i) * KB + qo[s]);
 #pragma unroll
-            for (int t = 0; t < ITEMS; ++t) issue(t, a, smb + a * BF_STG);
+        for (int j = 0; j < FN; ++j) b[j] = *(const i4v*)(S + Tl::SA + (rb + 32 * j) * KB + qo[s]);
+    };
+    auto mul = [&](const i4v (&a)[FM], const i4v (&b)[FN]) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    __builtin_bit_cast(bf8, a[i]), __builtin_bit_cast(bf8, b[j]), acc[i][j], 0, 0, 0);
+    };
+    if constexpr (FM * FN == 1) {
+        // one MFMA per k-step hides nothing: all of a chunk's reads up front
+        constexpr int AHEAD = NST - 1;
+#pragma unroll
+        for (int a = 0; a < AHEAD; ++a) issue(a, smb + a * Tl::STG);
+        int st = 0;
+        for (int c = 0; c < nch; ++c) {
+            // chunk c landed (the AHEAD - 1 chunks after it stay in flight), and
+            // every wave has read chunk c - 1, whose stage chunk c + AHEAD takes
+            __builtin_amdgcn_s_waitcnt(bf_vmcnt((AHEAD - 1) * ITEMS));
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            i4v ca[KS][FM], cb[KS][FN];
+#pragma unroll
+            for (int s = 0; s < KS; ++s) read(ca[s], cb[s], smb + st * Tl::STG, s);
+            issue(c + AHEAD, smb + (st == 0 ? NST - 1 : st - 1) * Tl::STG);
+#pragma unroll
+            for (int s = 0; s < KS; ++s) mul(ca[s], cb[s]);
+            st = st == NST - 1 ? 0 : st + 1;
         }
-    int st = 0;
-    for (int c = 0; c < nch; ++c) {
-        // chunk c landed: the chunks after it (at most AHEAD - 1) stay in flight
-        const int later = nch - 1 - c < AHEAD - 1 ? nch - 1 - c : AHEAD - 1;
-        if (later >= 2) __builtin_amdgcn_s_waitcnt(bf_vmcnt(2 * ITEMS));
-        else if (later == 1) __builtin_amdgcn_s_waitcnt(bf_vmcnt(ITEMS));
-        else __builtin_amdgcn_s_waitcnt(bf_vmcnt(0));
+    } else {
+        i4v fa[2][FM], fb[2][FN];                       // a k-step's operands, one step ahead
+#pragma unroll
+        for (int a = 0; a < NST; ++a) issue(a, smb + a * Tl::STG);
+        __builtin_amdgcn_s_waitcnt(bf_vmcnt((NST - 1) * ITEMS));
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        const char* S = smb + st * BF_STG;
-        char* NA = smb + (st == 0 ? BF_NST - 1 : st - 1) * BF_STG;   // (c + AHEAD) % NST: chunk c - 1's
-        const bool more = c + AHEAD < nch;
-        i4v fa[8], fb[8];
+        read(fa[0], fb[0], smb, 0);
+        int st = 0;
+        for (int c = 0; c < nch; ++c) {
+            char* const S = smb + st * Tl::STG;
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            fa[s] = *(const i4v*)(S + rda[s]);
-            fb[s] = *(const i4v*)(S + rdb[s]);
+            for (int s = 0; s < KS - 1; ++s) {
+                read(fa[(s + 1) & 1], fb[(s + 1) & 1], S, s + 1);
+                __builtin_amdgcn_sched_barrier(0);          // the next step's reads before this one's MFMAs
+                mul(fa[s & 1], fb[s & 1]);
+            }
+            // chunk c is in registers (everyone's): its stage takes chunk c + NST.
+            // Chunk c + 1 has landed once the NST - 2 chunks after it are all that
+            // is outstanding; the last step's MFMAs cover its first reads.
+            __builtin_amdgcn_s_waitcnt(bf_vmcnt((NST - 2) * ITEMS));
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            st = st == NST - 1 ? 0 : st + 1;
+            read(fa[0], fb[0], smb + st * Tl::STG, 0);
+            issue(c + NST, S);
+            __builtin_amdgcn_sched_barrier(0);
+            mul(fa[(KS - 1) & 1], fb[(KS - 1) & 1]);
         }
-        if (more) {                                      // its stage was read before this chunk
+    }
+    // epilogue: lane l, register e of block (i, j) <-> row 32 i + 8 (e / 4) +
+    // 4 (l / 32) + e % 4, column 32 j + l % 32 of the wave's part
 #pragma unroll
-            for (int t = 0; t < ITEMS; ++t) issue(t, c + AHEAD, NA);
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            const int n = n0 + (wn * FN + j) * 32 + r32;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int m = m0 + (wm * FM + i) * 32 + 8 * (e >> 2) + 4 * hq + (e & 3);
+                if (m < M && n < N) C[(long long)m * ldc + n] = acc[i][j][e];
+            }
         }
-#pragma unroll
-        for (int s = 0; s < 8; ++s)
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8, fa[s]),
-                                                          __builtin_bit_cast(bf8, fb[s]), acc, 0, 0, 0);
-        st = st == BF_NST - 1 ? 0 : st + 1;
-    }
-    // epilogue: lane l, register e <-> row m0 + 32wm + 8(e/4) + 4(l/32) + e%4, column n0 + 32wn + l%32
-    const int n = n0 + wn * 32 + r32;
-    if (n >= N) return;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const int m = m0 + wm * 32 + 8 * (e >> 2) + 4 * hq + (e & 3);
-        if (m < M) C[(long long)m * ldc + n] = acc[e];
-    }
+}
+
+template <int WM, int WN, int FM, int FN, int KB, int NST>
+bool launch_bf16(const unsigned short* Ab, const unsigned short* Bt, float* C, int M, int N, int Kp, int ldc,
+                 hipStream_t s) {
+    using Tl = BfTile<WM, WN, FM, FN, KB, NST>;
+    static_assert(Tl::LDS <= 160 * 1024, "LDS");
+    // set once per process, thread-safely, before any launch below
+    static const bool attr = [] {
+        (void)hipFuncSetAttribute((const void*)k_bf16mm<WM, WN, FM, FN, KB, NST>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, Tl::LDS);
+        return true;
+    }();
+    (void)attr;
+    const long long tiles = (long long)((M + Tl::BM - 1) / Tl::BM) * ((N + Tl::BN - 1) / Tl::BN);
+    ACFUN_LAUNCH("k_bf16mm", (k_bf16mm<WM, WN, FM, FN, KB, NST>), dim3((unsigned)((tiles + 7) / 8 * 8)),
+                 dim3(Tl::T), Tl::LDS, s, Ab, Bt, C, M, N, Kp, ldc, (unsigned)((long long)M * Kp * 2),
+                 (unsigned)((long long)N * Kp * 2));
+    return check_launch("k_bf16mm");
 }
 
 // C[0:M, 0:N] (row stride ldb = ldc) = bf16(A[0:M, :]) x bf16(B[:, 0:N]) on bf16 MFMA
@@ -241,18 +325,22 @@ bool bf16_region(int M, int N, int ldb, int K, const float* A, const float* B, f
     ACFUN_LAUNCH("k_pack_bf16", k_pack_bf16, dim3((unsigned)(nba + nbb)), dim3(256), 0, s, A, B, M, N, K, K, ldb, Kp,
                        (int)nba, ab.as<unsigned short>(), bt.as<unsigned short>(), va, vb);
     if (!check_launch("k_pack_bf16")) return false;
-    constexpr int lds = BF_NST * BF_STG;
-    // set once per process, thread-safely, before any launch below
-    static const bool attr = [&] {
-        (void)hipFuncSetAttribute((const void*)k_bf16mm, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        return true;
-    }();
-    (void)attr;
-    const long long tiles = (long long)((M + BF_BM - 1) / BF_BM) * ((N + BF_BN - 1) / BF_BN);
-    ACFUN_LAUNCH("k_bf16mm", k_bf16mm, dim3((unsigned)tiles), dim3(256), lds, s, ab.as<unsigned short>(),
-                 bt.as<unsigned short>(), C, M, N, Kp, ldb, (unsigned)((long long)M * Kp * 2),
-                 (unsigned)((long long)N * Kp * 2));
-    return check_launch("k_bf16mm");
+    const unsigned short *pa = ab.as<unsigned short>(), *pb = bt.as<unsigned short>();
+    // Tile by the time of the busiest CU, us, fitted to the sizes above: a tile
+    // costs 0.0040, 0.0090 alone on its CU (eight waves, three stages) or 0.0075
+    // beside another (four waves, two workgroups per CU), and 0.0262 per K.
+    auto per_cu = [&](int b) {
+        const long long t = (long long)((M + b - 1) / b) * ((N + b - 1) / b);
+        return (float)((t + num_cus() - 1) / num_cus());
+    };
+    const float n128 = per_cu(128), k = (float)Kp;
+    const float t64 = 3.f + per_cu(64) * k * 0.0040f;
+    const float t128 = 3.f + (n128 < 2.f ? k * 0.0090f : n128 * k * 0.0075f);
+    const float t256 = 4.f + per_cu(256) * k * 0.0262f;
+    if (t256 < t128 && t256 < t64) return launch_bf16<2, 4, 4, 2, 128, 2>(pa, pb, C, M, N, Kp, ldb, s);
+    if (t64 <= t128) return launch_bf16<2, 2, 1, 1, 256, 4>(pa, pb, C, M, N, Kp, ldb, s);
+    if (n128 < 2.f) return launch_bf16<2, 4, 2, 1, 128, 3>(pa, pb, C, M, N, Kp, ldb, s);
+    return launch_bf16<2, 2, 2, 2, 128, 2>(pa, pb, C, M, N, Kp, ldb, s);
 }
 
 }  // namespace

@@ -1,0 +1,33 @@
+"""acfun_gemm_bf16's tiles (64, 128 with one or several per CU, 256) at their
+edges: M and N that end 16 past a tile, K below, at and past a chunk, more
+stages than chunks.  Against the f64 product of the rounded operands (the
+16-aligned region; M and N are multiples of 16 here); the bound is fp32
+accumulation over K terms, sqrt(K) * 2^-24 on the output's scale, taken four
+times."""
+import numpy as np
+import pytest
+
+from tests.helpers import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (16, 16, 1), (80, 144, 128), (144, 80, 129), (272, 528, 640),        # 64
+    (1936, 2064, 384), (1040, 2064, 1100),                               # 128, one per CU
+    (3008, 2000, 300), (2064, 4112, 130),                                # 128, several per CU
+    (4080, 4000, 520), (4112, 3856, 1030),                               # 256
+])
+def test_bf16_tiles(gpu, rng, M, N, K):
+    torch = pytest.importorskip("torch")
+    g = torch.Generator().manual_seed(int(rng.integers(1 << 30)))
+    a, b = (torch.rand(s, generator=g) * 2 - 1 for s in ((M, K), (K, N)))
+    ta, tb = a.cuda(), b.cuda()
+    y = torch.full((M + 1, N), 7.0, device="cuda")        # one row past C stays untouched
+    torch.cuda.synchronize()
+    assert gpu.acfun_dev_gemm_bf16(M, N, K, ta.data_ptr(), tb.data_ptr(), y.data_ptr(), None) == 0
+    assert gpu.acfun_sync() == 0
+    want = a.bfloat16().double() @ b.bfloat16().double()
+    got = y.cpu()
+    assert rel_err(got[:M].numpy(), want.numpy()) < 4 * np.sqrt(K) * 2.0 ** -24 + 2.0 ** -22
+    assert bool((got[M] == 7.0).all())
