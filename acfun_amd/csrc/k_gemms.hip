@@ -26,7 +26,9 @@
 //   196 x 256 x 1024 GEMM         4.7   (16.5)    64 x 1000 x 2048 GEMM    7.4  (17.4)
 //   3x3 14 x 14 x 256, 1 image    7.5   (30.2)    3x3 7 x 7 x 512, 1 image 11.5 (59.9)
 //   3x3/2 14 x 14 x 512, 1 image  11.9  (84.0)    999 x 777 x 1333 GEMM    26.9 (57.5)
-//   3x3/2 28 x 28 x 256, 16 imgs  39.2  (47.1)    20001 x 131 x 259 GEMM   39.6 (58.0)
+//   3x3/2 28 x 28 x 256, 16 imgs  39.2  (47.1)    20001 x 131 x 259 GEMM   36.9 (58.3)
+//   3x3 20 x 20 x 30 -> 50, 2     5.3   (22.1)    3x3 21 x 21 x 248, 1     10.5 (28.7)
+//   7x7 28 x 28 x 12 -> 224, 9    29.2  (42.4)    3x3 51 x 51 x 143, 60   539   (708)
 #include "rt.hpp"
 
 namespace acfun {
@@ -58,12 +60,18 @@ __device__ __forceinline__ void ld(float (&d)[FN], __amdgpu_buffer_rsrc_t rsrc, 
     }
 }
 
-template <int FM, int FN, int W, bool CONV>
+// MODE GS_GEMM: a plain product.  GS_CONV: a convolution with Cin a multiple of
+// 16, a block within one tap.  GS_TAPS: any Cin; K is walked as KH KW taps of
+// Cin rounded up to 4 channels, so a lane's quad lies in one tap and each lane
+// follows its own (kh, kw, channel).
+enum { GS_GEMM, GS_CONV, GS_TAPS };
+template <int FM, int FN, int W, int MODE>
 __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, const float* __restrict__ B,
                                                   float* __restrict__ C, const float* __restrict__ bias,
                                                   const float* __restrict__ res, int M, int N, int K,
                                                   int lda, int ldb, int ldc, int ldr, int act, GsConv cv) {
     constexpr unsigned kOOB = 0x80000000u;
+    constexpr bool CONV = MODE != GS_GEMM, TAPS = MODE == GS_TAPS;
     constexpr int TM = 16 * FM, TN = 16 * FN, LDT = TN + 4;
     constexpr int D = FM * FN >= 16 ? 2 : FM * FN >= 4 ? 3 : 4;   // 16-k blocks in flight, as registers allow
     constexpr int NO = TM * TN / (64 * W) > 0 ? TM * TN / (64 * W) : 1;   // outputs per thread
@@ -114,7 +122,7 @@ __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, c
                 const int n = m / hw, rem = m - n * hw;
                 const int oh = rem / cv.OW, ow = rem - oh * cv.OW;
                 const int ih0 = oh * cv.stride - cv.pad, iw0 = ow * cv.stride - cv.pad;
-                cbase[i] = ((n * cv.H + ih0) * cv.W + iw0) * cv.Cin * 4 + 16 * lg;
+                cbase[i] = ((n * cv.H + ih0) * cv.W + iw0) * cv.Cin * 4 + (TAPS ? 0 : 16 * lg);
                 unsigned rm = 0, cm = 0;
                 for (int d = 0; d < 8; ++d) {
                     rm |= ((unsigned)(ih0 + d) < (unsigned)cv.H) ? (1u << d) : 0u;
@@ -132,7 +140,8 @@ __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, c
         vb[j] = n0 + FN * lr < N ? (unsigned)((4 * lg + j) * ldb + n0 + FN * lr) * 4u : kOOB;
 
     // this wave's 16-k blocks
-    const int nb = K >> 4;
+    const int cinp = (cv.Cin + 3) & ~3, ntap = TAPS ? K / cv.Cin : 0;   // GS_TAPS: channels walked, taps
+    const int nb = TAPS ? (ntap * cinp + 15) >> 4 : K >> 4;
     const int b0 = (int)((long long)wave * nb / W), n = (int)((long long)(wave + 1) * nb / W) - b0;
     // load cursor: the block's scalar offsets, CONV: its tap
     int cur = 0, ic = 0, kh = 0, kw = 0;
@@ -142,7 +151,12 @@ __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, c
 #pragma unroll
         for (int i = 0; i < FM; ++i) va[i] = (cmask[i] >> bit) & 1ull ? (unsigned)(cbase[i] + to) : kOOB;
     };
-    if (CONV) {
+    if (TAPS) {                                         // this lane's quad of block b0
+        const int k0 = 16 * b0 + 4 * lg, tap = k0 / cinp;
+        ic = k0 - tap * cinp;
+        kh = tap / cv.KW;
+        kw = tap - kh * cv.KW;
+    } else if (CONV) {
         const int k0 = 16 * b0, tap = k0 / cv.Cin;
         ic = k0 - tap * cv.Cin;
         kh = tap / cv.KW;
@@ -151,6 +165,29 @@ __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, c
         set_tap();
     }
     float a[D][FM][4], b[D][4][FN];
+    int left[TAPS ? D : 1];                             // GS_TAPS: the quad's channels inside Cin
+    const int bcol = n0 + FN * lr;
+    auto load_taps = [&](float (&as)[FM][4], float (&bs)[4][FN], int& lf) {
+        const int tap = kh * cv.KW + kw, bit = kh * 8 + kw;
+        const int to = ((kh * cv.W + kw) * cv.Cin + ic) * 4;
+        const unsigned rb = (unsigned)((tap * cv.Cin + ic) * ldb + bcol) * 4u;
+        const bool in = tap < ntap;
+        lf = in ? cv.Cin - ic : 0;
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+            ld<4>(as[i], ares, in && ((cmask[i] >> (bit & 63)) & 1ull) ? (unsigned)(cbase[i] + to) : kOOB, 0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            ld<FN>(bs[j], bres, j < lf && bcol < N ? rb + (unsigned)(j * ldb) * 4u : kOOB, 0);
+        if (cur + 1 < n) {
+            ++cur;
+            ic += 16;
+            while (ic >= cinp) {
+                ic -= cinp;
+                if (++kw == cv.KW) { kw = 0; ++kh; }
+            }
+        }
+    };
     auto load = [&](float (&as)[FM][4], float (&bs)[4][FN]) {
 #pragma unroll
         for (int i = 0; i < FM; ++i) ld<4>(as[i], ares, va[i], sa);
@@ -173,6 +210,12 @@ __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, c
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = f4s{0.f, 0.f, 0.f, 0.f};
+    auto clear = [&](float (&as)[FM][4], int lf) {      // channels past Cin: the next pixel's floats
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) as[i][e] = e < lf ? as[i][e] : 0.f;
+    };
     auto mul = [&](const float (&as)[FM][4], const float (&bs)[4][FN]) {
 #pragma unroll
         for (int k = 0; k < 4; ++k)
@@ -182,7 +225,26 @@ __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, c
                 for (int j = 0; j < FN; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(as[i][k], bs[k][j], acc[i][j], 0, 0, 0);
     };
-    if (n > 0) {
+    if constexpr (TAPS) {
+        if (n > 0) {
+            auto step = [&](float (&as)[FM][4], const float (&bs)[4][FN], int lf) {
+                if (cinp != cv.Cin) clear(as, lf);
+                mul(as, bs);
+            };
+#pragma unroll
+            for (int s = 0; s < D; ++s) load_taps(a[s], b[s], left[s]);
+            int done = 0;
+            for (; done + D <= n; done += D)
+#pragma unroll
+                for (int s = 0; s < D; ++s) {
+                    step(a[s], b[s], left[s]);
+                    load_taps(a[s], b[s], left[s]);
+                }
+#pragma unroll
+            for (int s = 0; s < D - 1; ++s)
+                if (done + s < n) step(a[s], b[s], left[s]);
+        }
+    } else if (n > 0) {
 #pragma unroll
         for (int s = 0; s < D; ++s) load(a[s], b[s]);
         int done = 0;
@@ -236,17 +298,19 @@ __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, c
     }
 }
 
-// The tiles and their cost, us: fixed + per_k * K for each tile the busiest CU
-// runs (one MFMA rate per shape: 16 x 16 and 16 x 32 are bound by the vector
-// loads, the others by MFMA and what latency its waves leave) + half a us per
-// further tile.  Fitted to sweeps over M, N, K of ResNet-50's layers at 1 to 64
-// images and of plain GEMMs; it is within 10 % of most of them.
-// 32 x 64 on two waves only pays with three or more workgroups a CU (1024^3,
-// 512 workgroups: 36 us -- they do not spread over the SIMDs).
-struct GsTile { int fm, fn, w, min_per_cu; float fixed, per_k; };
+// The tiles and their cost, us: fixed, then per_k * K for each tile the busiest
+// CU runs (16 x 16 and 16 x 32 are bound by the vector loads, the others by MFMA
+// and what latency their waves leave), and `each` for every tile after the
+// first (its set-up, first loads and LDS sum).  Fitted to sweeps over M, N, K of
+// ResNet-50's layers at 1 to 64 images, plain GEMMs, and convolutions of any
+// channel count; within 10 % of most of them.  32 x 64 on two waves only pays
+// with three or more workgroups a CU (1024^3, 512 workgroups: 36 us -- they do
+// not spread over the SIMDs), and 32 x 64 on four waves (three fit on a CU) loses
+// a round of workgroups past three (2000 x 999 x 333, four: 29 us against 19.5).
+struct GsTile { int fm, fn, w, min_per_cu; float fixed, per_k, each; };
 constexpr GsTile kGs[] = {
-    {1, 1, 4, 0, 3.0f, 0.0020f}, {1, 2, 4, 0, 3.0f, 0.0033f}, {1, 4, 4, 0, 3.3f, 0.0043f},
-    {2, 4, 4, 0, 3.8f, 0.0084f}, {2, 4, 2, 3, 4.0f, 0.0085f}, {4, 4, 8, 0, 5.0f, 0.0158f}};
+    {1, 1, 4, 0, 3.0f, 0.0020f, 0.5f}, {1, 2, 4, 0, 3.0f, 0.0033f, 0.55f}, {1, 4, 4, 0, 3.3f, 0.0043f, 0.75f},
+    {2, 4, 4, 0, 3.8f, 0.0084f, 1.0f}, {2, 4, 2, 3, 4.0f, 0.0085f, 1.5f},  {4, 4, 8, 0, 5.0f, 0.0158f, 4.0f}};
 constexpr int kGsN = sizeof(kGs) / sizeof(kGs[0]);
 
 long long tiles_of(long long M, long long N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
@@ -258,7 +322,8 @@ int pick(int M, int N, int K, float* us) {
         const GsTile& t = kGs[i];
         const long long cus = num_cus(), total = tiles_of(M, N, 16 * t.fm, 16 * t.fn);
         const float n = (float)((total + cus - 1) / cus);
-        const float e = t.fixed + n * t.per_k * (float)K + 0.5f * (n - 1.f);
+        const float e = t.fixed + n * t.per_k * (float)K + t.each * (n - 1.f) +
+                        (t.fm == 2 && t.w == 4 && n > 3.f ? 5.f : 0.f);
         if (total >= cus * t.min_per_cu && e < *us) { *us = e; best = i; }
     }
     return best;
@@ -269,48 +334,48 @@ int pick(int M, int N, int K, float* us) {
 // 64 x 64 tiles (up to one per CU: 4.1 + 0.0183 K with its two K groups from
 // K = 512 on; more: 0.0153 K per tile on the busiest CU, a convolution 0.0178, or 0.0169
 // from two per CU on); k_gemm_f32 with split-K 16 us and little per K (so a
-// K past some 6,000 on a handful of tiles stays there); k_gemm_f32 without
-// it loses everywhere (1.0 to 2.1 times as long at 16 shapes from 20 to 8,000
-// tiles); F(2,3) wins from about half a 64 x 64 tile per CU on (3x3 14 x 14 x 256:
+// K past some 6,000 on a handful of tiles stays there); k_gemm_f32 without it
+// 4 us + the larger of 0.068 K and its padded product at 55 TFLOP/s (3x3 over
+// 100 x 100 x 17 -> 33, 16 images: 64 us against 103 here); F(2,3) wins from about half a 64 x 64 tile per CU on (3x3 14 x 14 x 256:
 // 8 images, 100 tiles, 21.4 against 31.4 us; 12, 148 tiles, 31.7 against 32.4
 // with the filter transform; 16, 196 tiles, 41 against 33).  5 % in favour of
 // the other kernel.
-bool wins(int M, int N, int K, GsAlt alt) {
+bool wins(int M, int N, int K, GsAlt alt, float scale = 1.f) {
     const long long t = tiles_of(M, N, 64, 64), cus = num_cus();
-    if (alt == GsAlt::F32) return true;
     if (alt == GsAlt::WINO) return 2 * t <= cus;
-    if (t > 2 * cus) return false;
+    if (t > 2 * cus && alt != GsAlt::F32) return false;
     const float n = (float)((t + cus - 1) / cus), k = (float)K;
     float other;
     if (alt == GsAlt::SPLITK) other = 16.f + 0.0002f * k;
+    else if (alt == GsAlt::F32) other = 4.f + fmaxf(0.068f * k, (float)t * k * (2.f * 64 * 64 / 55e6f));
     else if (t <= cus) other = K >= 512 ? 4.1f + 0.0183f * k : 5.5f + 0.0177f * k;
     else other = 4.2f + n * k * (alt == GsAlt::G32 ? 0.0153f : t < 2 * cus ? 0.0178f : 0.0169f);
     float us;
     pick(M, N, K, &us);
-    return us < 0.95f * other;
+    return us * scale < 0.95f * other;
 }
 
-template <int FM, int FN, int W, bool CONV>
+template <int FM, int FN, int W, int MODE>
 bool launch(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C, int ldc,
             const float* bias, int act, hipStream_t s, const float* res, int ldr, const GsConv& cv) {
     const long long total = (long long)((M + 16 * FM - 1) / (16 * FM)) * ((N + 16 * FN - 1) / (16 * FN));
     const unsigned grid = (unsigned)((total + 7) / 8 * 8);
-    ACFUN_LAUNCH("k_gemms", (k_gemms<FM, FN, W, CONV>), dim3(grid), dim3(64 * W), 0, s, A, B, C, bias, res, M,
+    ACFUN_LAUNCH("k_gemms", (k_gemms<FM, FN, W, MODE>), dim3(grid), dim3(64 * W), 0, s, A, B, C, bias, res, M,
                  N, K, lda, ldb, ldc, ldr, act, cv);
     return check_launch("k_gemms");
 }
 
-template <bool CONV>
+template <int MODE>
 bool run(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
                  int ldc, const float* bias, int act, hipStream_t s, const float* res, int ldr, const GsConv& cv) {
     float us;
     switch (pick(M, N, K, &us)) {
-        case 0: return launch<1, 1, 4, CONV>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
-        case 1: return launch<1, 2, 4, CONV>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
-        case 2: return launch<1, 4, 4, CONV>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
-        case 3: return launch<2, 4, 4, CONV>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
-        case 4: return launch<2, 4, 2, CONV>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
-        default: return launch<4, 4, 8, CONV>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
+        case 0: return launch<1, 1, 4, MODE>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
+        case 1: return launch<1, 2, 4, MODE>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
+        case 2: return launch<1, 4, 4, MODE>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
+        case 3: return launch<2, 4, 4, MODE>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
+        case 4: return launch<2, 4, 2, MODE>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
+        default: return launch<4, 4, 8, MODE>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
     }
 }
 
@@ -323,14 +388,15 @@ bool gemms_wins(int M, int N, int K, int lda, int ldb, GsAlt alt) {
 
 bool gemms_f32(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C, int ldc,
                const float* bias, int act, hipStream_t s, const float* res, int ldr) {
-    return run<false>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, GsConv{});
+    return run<GS_GEMM>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, GsConv{});
 }
 
 bool convs_wins(const ConvShape& g, int Cout, GsAlt alt) {
     const long long M = (long long)g.N * g.OH * g.OW, K = (long long)g.KH * g.KW * g.Cin;
-    return M > 0 && K > 0 && Cout > 0 && g.Cin % 16 == 0 && g.KH <= 8 && g.KW <= 8 &&
+    return M > 0 && K > 0 && Cout > 0 && g.KH <= 8 && g.KW <= 8 &&
            (long long)g.N * g.H * g.W * g.Cin * 4 < 0x7fffffffll && K * Cout * 4 < 0x7fffffffll &&
-           M < 0x7fffffffll && tiles_of(M, Cout, 16, 16) < 0x7ffffff0ll && wins((int)M, Cout, (int)K, alt);
+           M < 0x7fffffffll && tiles_of(M, Cout, 16, 16) < 0x7ffffff0ll &&
+           wins((int)M, Cout, (int)K, alt, g.Cin % 16 ? 1.25f : 1.f);   // GS_TAPS: address work per block
 }
 
 bool convs_f32(const ConvShape& g, const float* in, const float* w, const float* bias, int Cout, float* out,
@@ -338,7 +404,9 @@ bool convs_f32(const ConvShape& g, const float* in, const float* w, const float*
     const GsConv cv{g.H, g.W, g.Cin, g.KW, g.stride, g.pad, g.OH, g.OW,
                     (unsigned)((long long)g.N * g.H * g.W * g.Cin * 4)};
     const int M = g.N * g.OH * g.OW, K = g.KH * g.KW * g.Cin;
-    return run<true>(M, Cout, K, in, g.Cin, w, Cout, out, Cout, bias, act, s, res, ldr, cv);
+    if (g.Cin % 16 == 0)
+        return run<GS_CONV>(M, Cout, K, in, g.Cin, w, Cout, out, Cout, bias, act, s, res, ldr, cv);
+    return run<GS_TAPS>(M, Cout, K, in, g.Cin, w, Cout, out, Cout, bias, act, s, res, ldr, cv);
 }
 
 }  // namespace acfun

@@ -195,8 +195,7 @@ bool conv32_f32(const ConvShape& g, const float* in, const float* w, const float
                 float* out, int act, hipStream_t s, const float* res = nullptr, int ldr = 0);
 // Few output tiles, or operands of any alignment (k_gemms.hip): small tiles
 // whose K range a workgroup's waves split.  gemms_wins / convs_wins say whether
-// the shape is admitted (a convolution: Cin a multiple of 16, KH and KW <= 8)
-// and this is the faster kernel than `alt`, the one it would otherwise run.
+// the shape is admitted (a convolution: KH and KW <= 8) and this is the faster kernel than `alt`, the one it would otherwise run.
 enum class GsAlt { G32, CONV32, F32, SPLITK, WINO };
 bool gemms_wins(int M, int N, int K, int lda, int ldb, GsAlt alt);
 bool gemms_f32(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,

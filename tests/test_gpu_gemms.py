@@ -52,7 +52,11 @@ def test_gemm_small_tiles(gpu, rng, M, N, K, off):
 @pytest.mark.parametrize("N,H,W,Cin,ks,Cout,s,p", [
     (1, 14, 14, 256, 3, 256, 1, 1), (1, 7, 7, 512, 3, 512, 1, 1), (2, 9, 11, 16, 3, 20, 1, 1),
     (1, 14, 14, 512, 3, 512, 2, 1), (3, 13, 10, 48, 5, 33, 2, 2), (1, 28, 28, 512, 1, 100, 2, 0),
-    (16, 57, 30, 80, 3, 80, 2, 1), (1, 3, 3, 16, 3, 4, 1, 1), (2, 12, 12, 32, 8, 24, 3, 4)])
+    (16, 57, 30, 80, 3, 80, 2, 1), (1, 3, 3, 16, 3, 4, 1, 1), (2, 12, 12, 32, 8, 24, 3, 4),
+    # any channel count: taps padded to 4 channels, several taps in a 16-deep block
+    (1, 9, 8, 1, 3, 5, 2, 1), (2, 13, 11, 3, 5, 17, 2, 2), (1, 14, 9, 5, 4, 7, 3, 0),
+    (1, 45, 10, 248, 3, 32, 1, 1), (1, 24, 11, 28, 7, 32, 2, 3), (3, 12, 7, 37, 3, 33, 1, 1),
+    (2, 9, 9, 143, 1, 20, 2, 0), (1, 10, 10, 12, 8, 64, 1, 4)])
 def test_conv_small_tiles(gpu, rng, N, H, W, Cin, ks, Cout, s, p):
     torch = pytest.importorskip("torch")
     x = rng.uniform(0, 1, (N, H, W, Cin)).astype(np.float32)
