@@ -544,7 +544,7 @@ __global__ __launch_bounds__(256) void k_gconv4_3x3(const float* __restrict__ in
 }
 
 // Depthwise 3x3 / stride 2 + activation + 3x3 / stride-2 MaxPool, row-streaming
-// form: a lane owns 4 channels of one pooled column and walks a strip of RP
+// form: a lane owns 4 channels of one pooled column and walks a strip of rp
 // pooled rows down the image.  Per depthwise row y it loads the two new input
 // rows (7 columns: those of depthwise columns 2 pw - pp .. 2 pw - pp + 2), and
 // keeps only running sums: the depthwise accumulators of row y + 1 started
@@ -555,11 +555,10 @@ __global__ __launch_bounds__(256) void k_gconv4_3x3(const float* __restrict__ in
 // k_dwconv3_blk then k_maxpool3s2_row.  No LDS, no barriers: lanes stream
 // independently, and workgroups are XCD-ordered so the strips that share
 // input rows read them through one L2.
-constexpr int DWR_RP = 4;                               // pooled rows per strip
 __global__ __launch_bounds__(256) void k_dwconv3_pool_rs(
     const float* __restrict__ in, int H, int W, int C4, const float* __restrict__ w,
     const float* __restrict__ bias, int pad, int OH, int OW, int act, int PP, int PH, int PW,
-    int nstrip, int items, int in_bytes, int pvec_end, float4* __restrict__ out, int post_relu) {
+    int nstrip, int rp, int items, int in_bytes, int pvec_end, float4* __restrict__ out, int post_relu) {
     constexpr unsigned kOOB = 0x80000000u;
     const int per = (int)(gridDim.x >> 3);
     const int blk = (int)(blockIdx.x & 7u) * per + (int)(blockIdx.x >> 3);
@@ -572,7 +571,7 @@ __global__ __launch_bounds__(256) void k_dwconv3_pool_rs(
     const int t = idx / lps;
     const int st = t % nstrip;
     const int n = t / nstrip;
-    const int ph0 = st * DWR_RP, ph1 = ph0 + DWR_RP < PH ? ph0 + DWR_RP : PH;
+    const int ph0 = st * rp, ph1 = ph0 + rp < PH ? ph0 + rp : PH;
     const int c = 4 * q;
     float wk[4][9];
     {
@@ -1225,12 +1224,22 @@ bool dwconv_pool_f32(const float* in, int N, int H, int W, int C, const float* w
     const int pvec_end = C >= 16 ? (C & ~15) : (C >= 8 ? (C & ~7) : 0);
     const long long in_bytes = (long long)N * H * W * C * 4;
     if (stride == 2 && in_bytes < (1ll << 31)) {
-        const int nstrip = (PH + DWR_RP - 1) / DWR_RP;
-        const long long lanes = (long long)N * nstrip * ((PW * C4 + 63) / 64 * 64);
+        // Pooled rows per strip.  A strip is a chain of one memory round trip per
+        // depthwise row, so four rows a strip only once the lanes fill the chip
+        // (two waves per SIMD): shorter strips re-read more halo rows (4 rows is
+        // best from there on: 32 x 112 x 112 x 96 takes 32.5 us, 2 or 3 rows 39
+        // to 43), but below it only the chain's length counts.  Before / after:
+        // 18 x 58 x 17 x 16 19.5 / 8.2 us, 1 x 112 x 112 x 64 19.7 / 8.5,
+        // 8 x 112 x 112 x 96 24.8 / 14.2, 4 x 60 x 90 x 200 23.9 / 11.2.
+        const long long row = (PW * C4 + 63) / 64 * 64;
+        int rp = 4;
+        while (rp > 1 && (long long)N * ((PH + rp - 1) / rp) * row < 2ll * 4 * 64 * num_cus()) --rp;
+        const int nstrip = (PH + rp - 1) / rp;
+        const long long lanes = (long long)N * nstrip * row;
         const long long wgs = (lanes + 255) / 256;
         if (lanes < (1ll << 30)) {
             ACFUN_LAUNCH("k_dwconv_pool", k_dwconv3_pool_rs, dim3((unsigned)(8 * ((wgs + 7) / 8))), dim3(256),
-                         0, s, in, H, W, C4, w, bias, pad, OH, OW, act, ppad, PH, PW, nstrip, (int)lanes,
+                         0, s, in, H, W, C4, w, bias, pad, OH, OW, act, ppad, PH, PW, nstrip, rp, (int)lanes,
                          (int)in_bytes, pvec_end, (float4*)out, post_relu);
             return check_launch("k_dwconv3_pool_rs");
         }

@@ -184,3 +184,15 @@ def test_g_maxpool_nan(gpu, rng):
     for act, pr in ((0, 0), (1, 1)):
         assert_bitexact(run_gpool(gpu, x, w, b, 48, 1, 1, 6, act, 1, pr),
                         want_gpool(x, w, b, 48, 1, 1, 6, act, 1, pr), f"gconv NaN act={act}")
+
+
+@pytest.mark.parametrize("N,H,W,C", [(1, 58, 17, 16), (6, 58, 40, 64), (24, 58, 56, 64),
+                                     (40, 57, 57, 64), (1, 7, 8, 4)])
+def test_dw_maxpool_strip_heights(gpu, rng, N, H, W, C):
+    """Stride 2 from a handful of lanes to a full chip: strips of 1 to 4 rows."""
+    x = rng.standard_normal((N, H, W, C)).astype(np.float32)
+    x[0, H // 2, W // 2, 1] = np.nan
+    w = (rng.standard_normal((C, 3, 3)) * 0.3).astype(np.float32)
+    b = (rng.standard_normal(C) * 0.1).astype(np.float32)
+    assert_bitexact(run_dwpool(gpu, x, w, b, 2, 1, 1, 1, 0), want_dwpool(x, w, b, 2, 1, 1, 1, 0),
+                    f"dw+pool {N, H, W, C}")
