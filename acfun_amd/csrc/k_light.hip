@@ -554,15 +554,18 @@ __global__ __launch_bounds__(256) void k_gconv4_3x3(const float* __restrict__ in
 // out-of-range taps skipped by selects, so the result is bit for bit
 // k_dwconv3_blk then k_maxpool3s2_row.  No LDS, no barriers: lanes stream
 // independently, and workgroups are XCD-ordered so the strips that share
-// input rows read them through one L2.
-__global__ __launch_bounds__(256) void k_dwconv3_pool_rs(
+// input rows read them through one L2.  One wave per workgroup: the strips of a
+// full chip are some 9.6 waves per CU, which 256-thread workgroups rounded up to
+// 12 on half the CUs (32 x 112 x 112 x 96, inputs in HBM: 43.9 -> 42.7 us; 8
+// images 14.2 -> 13.4).
+__global__ __launch_bounds__(64) void k_dwconv3_pool_rs(
     const float* __restrict__ in, int H, int W, int C4, const float* __restrict__ w,
     const float* __restrict__ bias, int pad, int OH, int OW, int act, int PP, int PH, int PW,
     int nstrip, int rp, int items, int in_bytes, int pvec_end, float4* __restrict__ out, int post_relu) {
     constexpr unsigned kOOB = 0x80000000u;
     const int per = (int)(gridDim.x >> 3);
     const int blk = (int)(blockIdx.x & 7u) * per + (int)(blockIdx.x >> 3);
-    const int idx = blk * 256 + (int)threadIdx.x;
+    const int idx = blk * 64 + (int)threadIdx.x;
     if (idx >= items) return;
     // a strip's lanes are padded to whole waves, so every wave walks one way
     const int lps = (PW * C4 + 63) & ~63, li = idx % lps;
@@ -647,7 +650,7 @@ __global__ __launch_bounds__(256) void k_dwconv3_pool_rs(
         // its activated values go to a per-lane ring of the last three rows in
         // LDS, and pool row ph is formed, in kh order, once its top row 2 ph - PP
         // arrives.  Same arithmetic in the same order as the downward walk.
-        __shared__ f4 ring[9][256];
+        __shared__ f4 ring[9][64];
         const int lt = (int)threadIdx.x;
         f4 r2[7];
         bool ok2 = ldrow(2 * yB - pad + 2, r2);
@@ -1236,9 +1239,9 @@ bool dwconv_pool_f32(const float* in, int N, int H, int W, int C, const float* w
         while (rp > 1 && (long long)N * ((PH + rp - 1) / rp) * row < 2ll * 4 * 64 * num_cus()) --rp;
         const int nstrip = (PH + rp - 1) / rp;
         const long long lanes = (long long)N * nstrip * row;
-        const long long wgs = (lanes + 255) / 256;
+        const long long wgs = (lanes + 63) / 64;
         if (lanes < (1ll << 30)) {
-            ACFUN_LAUNCH("k_dwconv_pool", k_dwconv3_pool_rs, dim3((unsigned)(8 * ((wgs + 7) / 8))), dim3(256),
+            ACFUN_LAUNCH("k_dwconv_pool", k_dwconv3_pool_rs, dim3((unsigned)(8 * ((wgs + 7) / 8))), dim3(64),
                          0, s, in, H, W, C4, w, bias, pad, OH, OW, act, ppad, PH, PW, nstrip, rp, (int)lanes,
                          (int)in_bytes, pvec_end, (float4*)out, post_relu);
             return check_launch("k_dwconv3_pool_rs");
