@@ -315,12 +315,14 @@ constexpr int kGsN = sizeof(kGs) / sizeof(kGs[0]);
 
 long long tiles_of(long long M, long long N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
-int pick(int M, int N, int K, float* us) {
+// (cus: num_cus(), asked once per call -- it is a runtime call each time, and
+// one per entry of this table made the smallest products 0.5 us slower)
+int pick(int M, int N, int K, long long cus, float* us) {
     int best = 0;
     *us = 1e30f;
     for (int i = 0; i < kGsN; ++i) {
         const GsTile& t = kGs[i];
-        const long long cus = num_cus(), total = tiles_of(M, N, 16 * t.fm, 16 * t.fn);
+        const long long total = tiles_of(M, N, 16 * t.fm, 16 * t.fn);
         const float n = (float)((total + cus - 1) / cus);
         const float e = t.fixed + n * t.per_k * (float)K + t.each * (n - 1.f) +
                         (t.fm == 2 && t.w == 4 && n > 3.f ? 5.f : 0.f);
@@ -351,7 +353,7 @@ bool wins(int M, int N, int K, GsAlt alt, float scale = 1.f) {
     else if (t <= cus) other = K >= 512 ? 4.1f + 0.0183f * k : 5.5f + 0.0177f * k;
     else other = 4.2f + n * k * (alt == GsAlt::G32 ? 0.0153f : t < 2 * cus ? 0.0178f : 0.0169f);
     float us;
-    pick(M, N, K, &us);
+    pick(M, N, K, cus, &us);
     return us * scale < 0.95f * other;
 }
 
@@ -369,7 +371,7 @@ template <int MODE>
 bool run(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
                  int ldc, const float* bias, int act, hipStream_t s, const float* res, int ldr, const GsConv& cv) {
     float us;
-    switch (pick(M, N, K, &us)) {
+    switch (pick(M, N, K, num_cus(), &us)) {
         case 0: return launch<1, 1, 4, MODE>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
         case 1: return launch<1, 2, 4, MODE>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
         case 2: return launch<1, 4, 4, MODE>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
