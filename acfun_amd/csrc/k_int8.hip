@@ -489,11 +489,83 @@ __device__ void prep_row(const int8_t* __restrict__ wq, int taps, int Cin, int C
     if (threadIdx.x == 0) Sw[n] = red[0] + red[1] + red[2] + red[3];
 }
 
+// The same for kPrepCols = 4 output channels per block: a thread reads four
+// channels of four rows (a dword each, at any alignment), transposes them in
+// registers and writes one dword per channel.
+constexpr int kPrepCols = 4;
+__device__ void prep_cols(const int8_t* __restrict__ wq, int taps, int Cin, int Cinp, int N,
+                          int8_t* __restrict__ Bt, int ldb, int* __restrict__ Sw, int blk) {
+    const int n0 = blk * kPrepCols, nc = N - n0 < kPrepCols ? N - n0 : kPrepCols;
+    int sum[kPrepCols] = {0, 0, 0, 0};
+#pragma unroll 2
+    for (int k0 = 4 * threadIdx.x; k0 < ldb; k0 += 1024) {      // (ldb is a multiple of 128)
+        int tap = k0 / Cinp, ic = k0 - tap * Cinp;
+        unsigned r[4];
+        long long off[4];                                       // -1: a zero row
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            off[e] = tap < taps && ic < Cin ? ((long long)tap * Cin + ic) * N + n0 : -1;
+            if (++ic == Cinp) { ic = 0; ++tap; }
+        }
+        if (nc == kPrepCols) {                                  // (no branch per row: four loads in flight)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) __builtin_memcpy(&r[e], wq + (off[e] < 0 ? 0 : off[e]), 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[e] = off[e] < 0 ? 0u : r[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                r[e] = 0;
+                for (int c = 0; off[e] >= 0 && c < nc; ++c) r[e] |= (unsigned)(uint8_t)wq[off[e] + c] << (8 * c);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < kPrepCols; ++c) {
+            unsigned v = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const unsigned byte = (r[e] >> (8 * c)) & 0xffu;
+                v |= byte << (8 * e);
+                sum[c] += (int8_t)byte;
+            }
+            if (c < nc) *(unsigned*)(Bt + (long long)(n0 + c) * ldb + k0) = v;
+        }
+    }
+    __shared__ int red[4][kPrepCols];
+#pragma unroll
+    for (int c = 0; c < kPrepCols; ++c) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) sum[c] += __shfl_xor(sum[c], o);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][c] = sum[c];
+    }
+    __syncthreads();
+    const int c = threadIdx.x;
+    if (c < nc) Sw[n0 + c] = red[0][c] + red[1][c] + red[2][c] + red[3][c];
+}
+
+// Which of the two, for a K x N matrix.  Large ones are bound by the strided
+// reads, one cache line for each byte (3x3 x 512 -> 512, one 14 x 14 image: 29.8
+// us a call by single channels, 25.4 by fours); small ones by one block's walk
+// over K, and there a block per channel is four times the blocks (3x3 x 128 ->
+// 128, 32 x 28 x 28: 24.4 against 25.4).  At 3x3 x 256 -> 256 both take the same.
+constexpr long long kPrepBig = 1 << 20;
+__device__ __host__ inline bool prep_by4(int taps, int Cin, int N) {
+    return N >= 128 && (long long)taps * Cin * N >= kPrepBig;   // (N: at least 32 blocks)
+}
+inline unsigned prep_blocks(int taps, int Cin, int N) {
+    return prep_by4(taps, Cin, N) ? (unsigned)((N + kPrepCols - 1) / kPrepCols) : (unsigned)N;
+}
+__device__ void prep_block(const int8_t* __restrict__ wq, int taps, int Cin, int Cinp, int N,
+                           int8_t* __restrict__ Bt, int ldb, int* __restrict__ Sw, int blk) {
+    if (prep_by4(taps, Cin, N)) prep_cols(wq, taps, Cin, Cinp, N, Bt, ldb, Sw, blk);
+    else prep_row(wq, taps, Cin, Cinp, N, Bt, ldb, Sw, blk);
+}
+
 __global__ __launch_bounds__(256) void k_prep_weights(const int8_t* __restrict__ wq, int taps,
                                                       int Cin, int Cinp, int N,
                                                       int8_t* __restrict__ Bt, int ldb,
                                                       int* __restrict__ Sw) {
-    prep_row(wq, taps, Cin, Cinp, N, Bt, ldb, Sw, blockIdx.x);
+    prep_block(wq, taps, Cin, Cinp, N, Bt, ldb, Sw, blockIdx.x);
 }
 
 __global__ __launch_bounds__(256) void k_absmax_part(const float* __restrict__ x, size_t n,
@@ -502,7 +574,7 @@ __global__ __launch_bounds__(256) void k_absmax_part(const float* __restrict__ x
 }
 
 // The activation absmax (blocks < nb) and, in the same launch, the per-call
-// weight preparation (one block per output channel after them).
+// weight preparation (prep_blocks() blocks after them).
 __global__ __launch_bounds__(256) void k_absmax_prep(const float* __restrict__ x, size_t n,
                                                      float* __restrict__ part, int nb,
                                                      const int8_t* __restrict__ wq, int taps,
@@ -510,7 +582,7 @@ __global__ __launch_bounds__(256) void k_absmax_prep(const float* __restrict__ x
                                                      int8_t* __restrict__ Bt, int ldb,
                                                      int* __restrict__ Sw) {
     if ((int)blockIdx.x < nb) absmax_block(x, n, part, blockIdx.x, nb);
-    else prep_row(wq, taps, Cin, Cinp, N, Bt, ldb, Sw, blockIdx.x - nb);
+    else prep_block(wq, taps, Cin, Cinp, N, Bt, ldb, Sw, blockIdx.x - nb);
 }
 
 // acfun_quantize_weights (src/conv_int8.cpp:24-37): one lane per column.
@@ -811,7 +883,8 @@ bool alloc_weights(int taps, int Cinp, int N, hipStream_t s, PrepW& w) {
 }
 bool prep_weights(const int8_t* wq, int taps, int Cin, int Cinp, int N, hipStream_t s, PrepW& w) {
     if (!alloc_weights(taps, Cinp, N, s, w)) return false;
-    ACFUN_LAUNCH("k_prep_weights", k_prep_weights, dim3(N), dim3(256), 0, s, wq, taps, Cin, Cinp, N,
+    ACFUN_LAUNCH("k_prep_weights", k_prep_weights, dim3(prep_blocks(taps, Cin, N)), dim3(256), 0, s, wq, taps,
+                       Cin, Cinp, N,
                        w.bt.as<int8_t>(), w.ldb, w.sw.as<int>());
     return check_launch("k_prep_weights");
 }
@@ -968,8 +1041,9 @@ bool conv2d_int8_run(const float* in, const ConvShape& g, const int8_t* wq, cons
                 part = (float*)ar.get((size_t)kParts * sizeof(float));
                 if (!part) return false;
             }
-            if (nb + (prepared ? 0 : Cout) > 0) {
-                ACFUN_LAUNCH("k_absmax_prep", k_absmax_prep, dim3(nb + (prepared ? 0 : Cout)), dim3(256), 0, s,
+            const int np = prepared ? 0 : (int)prep_blocks(1, g.Cin, Cout);
+            if (nb + np > 0) {
+                ACFUN_LAUNCH("k_absmax_prep", k_absmax_prep, dim3(nb + np), dim3(256), 0, s,
                              in, inN, part, nb, wq, 1, g.Cin, Cinp, Cout, nbt, ldb, nsw);
                 if (!check_launch("k_absmax_prep")) return false;
             }
@@ -1002,8 +1076,9 @@ bool conv2d_int8_run(const float* in, const ConvShape& g, const int8_t* wq, cons
         // absmax pass is skipped and the quantizer reads that one "partial".
         int nb = amax_in || reuse ? 0 : (int)((n4 + 1023) / 1024);
         if (!amax_in && !reuse) nb = nb < 1 ? 1 : (nb > kParts ? kParts : nb);
-        if (nb + (prepared ? 0 : Cout) > 0) {
-            ACFUN_LAUNCH("k_absmax_prep", k_absmax_prep, dim3(nb + (prepared ? 0 : Cout)), dim3(256), 0, s, in,
+        const int np = prepared ? 0 : (int)prep_blocks(g.KH * g.KW, g.Cin, Cout);
+        if (nb + np > 0) {
+            ACFUN_LAUNCH("k_absmax_prep", k_absmax_prep, dim3(nb + np), dim3(256), 0, s, in,
                                inN, part, nb, wq, g.KH * g.KW, g.Cin, Cinp, Cout, nbt, ldb, nsw);
             if (!check_launch("k_absmax_prep")) return false;
         }
@@ -1049,7 +1124,8 @@ bool conv2d_int8_run(const float* in, const ConvShape& g, const int8_t* wq, cons
         return false;
     }
     if (!prepared) {
-        ACFUN_LAUNCH("k_prep_weights", k_prep_weights, dim3(Cout), dim3(256), 0, s, wq, g.KH * g.KW, g.Cin,
+        ACFUN_LAUNCH("k_prep_weights", k_prep_weights, dim3(prep_blocks(g.KH * g.KW, g.Cin, Cout)),
+                           dim3(256), 0, s, wq, g.KH * g.KW, g.Cin,
                            Cinp, Cout, nbt, ldb, nsw);
         if (!check_launch("k_prep_weights")) return false;
     }
@@ -1231,7 +1307,8 @@ bool conv2d_int8_q8_dev(const int8_t* q, int ldq_in, const float* s_in, const Co
         int8_t* nbt = (int8_t*)ar.get((size_t)Cout * ldb);
         int* nsw = (int*)ar.get((size_t)Cout * sizeof(int));
         if (!nbt || !nsw) return false;
-        ACFUN_LAUNCH("k_prep_weights", k_prep_weights, dim3(Cout), dim3(256), 0, s, wq, g.KH * g.KW, g.Cin,
+        ACFUN_LAUNCH("k_prep_weights", k_prep_weights, dim3(prep_blocks(g.KH * g.KW, g.Cin, Cout)),
+                           dim3(256), 0, s, wq, g.KH * g.KW, g.Cin,
                            Cinp, Cout, nbt, ldb, nsw);
         if (!check_launch("k_prep_weights")) return false;
         bt = nbt; sw = nsw;
@@ -1335,7 +1412,7 @@ bool i8_prepare(const int8_t* wq, int taps, int Cin, int N, I8Weights& w, hipStr
         return false;
     }
     w.taps = taps; w.Cin = Cin; w.N = N;
-    ACFUN_LAUNCH("k_prep_weights", k_prep_weights, dim3(N), dim3(256), 0, s, wq, taps, Cin, Cinp, N, w.bt,
+    ACFUN_LAUNCH("k_prep_weights", k_prep_weights, dim3(prep_blocks(taps, Cin, N)), dim3(256), 0, s, wq, taps, Cin, Cinp, N, w.bt,
                        w.ldb, w.sw);
     return check_launch("k_prep_weights");
 }

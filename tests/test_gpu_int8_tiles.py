@@ -1,6 +1,6 @@
 """int8 convolutions at tile counts where the launch shape changes: counts that
-are no multiple of 8 (workgroups without a tile) up to three per CU and past it.
-Integer sums and specified roundings: bit-exact against the oracle."""
+are no multiple of 8 (workgroups without a tile) up to three per CU and past it, and
+weight matrices either side of the preparation's two forms.  Integer sums and specified roundings: bit-exact against the oracle."""
 import ctypes as C
 
 import numpy as np
@@ -20,6 +20,9 @@ CASES = [  # N, H, W, Cin, Cout, ks, stride, act
     (1, 65, 63, 32, 65, 1, 1, 0),     # 130 of them, one live column in half
     (5, 57, 56, 24, 128, 3, 1, 1),    # 500
     (1, 112, 113, 40, 250, 1, 1, 1),  # 792: past three per CU
+    (1, 7, 7, 512, 230, 3, 1, 1),     # 2^20 weights and more: four channels per
+    (1, 6, 5, 1031, 1023, 1, 1, 0),   # preparation block, the last block ragged
+    (1, 5, 4, 700, 168, 3, 2, 1),     # (1,058,400 of them; 168 / 4 is whole)
 ]
 
 
@@ -41,3 +44,15 @@ def test_conv_int8_tile_counts(N, H, W, Cin, Cout, ks, stride, act, zero):
                                  0.0, p(got), act)
     want = oracle.conv2d_int8(x, wq, ws, b, ks, ks, Cout, stride, pad, act)
     assert np.array_equal(got, want), capi.last_error()
+
+
+@pytest.mark.parametrize("K,N", [(4096, 256), (4095, 256), (4099, 259), (8192, 128), (8256, 127)])
+def test_gemm_int8_prepared_by_fours(K, N):
+    """The weight preparation of a plain product: rows, not taps, to the dword."""
+    rng = np.random.default_rng(K + N)
+    A = rng.integers(0, 256, (3, K)).astype(np.uint8)
+    B = rng.integers(-128, 128, (K, N)).astype(np.int8)
+    got = np.full((3, N), -1, np.int32)
+    p = lambda a: C.c_void_p(a.ctypes.data)  # noqa: E731
+    capi.lib().acfun_gemm_int8(3, N, K, p(A), p(B), p(got))
+    assert np.array_equal(got, oracle.gemm_int8(A, B)), capi.last_error()
