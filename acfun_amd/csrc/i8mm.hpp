@@ -748,6 +748,7 @@ __global__ __launch_bounds__(256) void k_i8mm(I8M p) {
             p.amax[blockIdx.x] = mm;
         }
     }
+    __builtin_amdgcn_s_waitcnt(vmcnt_enc(0));           // the out-of-range loads, still on their way to LDS
 }
 
 

@@ -283,6 +283,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_bf16mm(const unsigned short* _
                 if (m < M && n < N) C[(long long)m * ldc + n] = acc[i][j][e];
             }
         }
+    __builtin_amdgcn_s_waitcnt(bf_vmcnt(0));            // the chunks issued past the end, still on their way to LDS
 }
 
 template <int WM, int WN, int FM, int FN, int KB, int NST>
