@@ -167,10 +167,6 @@ __global__ __launch_bounds__(64 * WM * WN) void k_bf16mm(const unsigned short* _
     const int rin = L - grp * GRP * gn;
     const int m0 = (grp * GRP + rin % rows) * BM, n0 = (rin / rows) * BN;
     const int nch = Kp / (KB / 2);
-    const __amdgpu_buffer_rsrc_t ares =
-        __builtin_amdgcn_make_buffer_rsrc((void*)Ab, (short)0, (int)a_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t bres =
-        __builtin_amdgcn_make_buffer_rsrc((void*)Bt, (short)0, (int)b_bytes, 0x00020000);
     // quad q of row r sits at slot q ^ sw(r): 8 consecutive rows' reads of one
     // quad cover all banks
     auto sw = [](int r) { return QR >= 8 ? r & (QR - 1) : (r >> 1) & (QR - 1); };
@@ -186,10 +182,16 @@ __global__ __launch_bounds__(64 * WM * WN) void k_bf16mm(const unsigned short* _
         const int row = RPI * (wave + NW * t) + rl, q = sl ^ sw(row);
         bv[t] = n0 + row < N ? (unsigned)((n0 + row) * Kp * 2 + 16 * q) : kOOB;
     }
-    // Every iteration issues one chunk (past the end the last one again, into a
-    // stage that is not read), so all waits of the loop are the same.
+    // Every iteration issues one chunk, so all waits of the loop are the same; past
+    // the last one out of range (an empty buffer): no memory traffic, and zeros to
+    // a stage whose contents are not multiplied.
     auto issue = [&](int c, char* st) {
-        const unsigned so = (unsigned)(c < nch ? c : nch - 1) * KB;
+        const bool live = c < nch;
+        const unsigned so = live ? (unsigned)c * KB : 0u;
+        const __amdgpu_buffer_rsrc_t ares =
+            __builtin_amdgcn_make_buffer_rsrc((void*)Ab, (short)0, live ? (int)a_bytes : 0, 0x00020000);
+        const __amdgpu_buffer_rsrc_t bres =
+            __builtin_amdgcn_make_buffer_rsrc((void*)Bt, (short)0, live ? (int)b_bytes : 0, 0x00020000);
 #pragma unroll
         for (int t = 0; t < AIT; ++t) bf_dma16(ares, st + (wave + NW * t) * 1024, av[t], so);
 #pragma unroll
