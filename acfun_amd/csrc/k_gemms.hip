@@ -7,8 +7,12 @@
 // one LDS round trip per chunk.  Here a tile is as small as 16 x 16, so the
 // tiles fill the CUs, and the W waves of a workgroup split K between them: wave
 // w takes a contiguous run of 16-deep blocks, and the partial tiles are summed
-// through LDS in wave order at the end (a shorter fp32 chain than one wave's:
-// the results are closer to the f64 product, not further).
+// through LDS in wave order at the end.  A chain of fp32 sums grows the rounding
+// error with the root of its length, so a wave adds its accumulators to its part
+// of LDS every 256 k or less and starts again from zero: K split between four
+// waves alone made chains of K / 4, longer than the K / 256 workgroups of the
+// split-K kernel (relative error, 1 to 64 rows, K = 2048: 4.06e-7, with the folds
+// 2.95e-7, split-K 2.95e-7; K = 6144: 7.0e-7, 2.95e-7, 3.0e-7).
 //
 // The waves share no operand, so there is no LDS staging and no barrier in the
 // loop: a lane loads its MFMA operands straight from memory, D blocks ahead.
@@ -65,8 +69,17 @@ __device__ __forceinline__ void ld(float (&d)[FN], __amdgpu_buffer_rsrc_t rsrc, 
 // Cin rounded up to 4 channels, so a lane's quad lies in one tap and each lane
 // follows its own (kh, kw, channel).
 enum { GS_GEMM, GS_CONV, GS_TAPS };
+// Waves per SIMD the registers must leave room for.  Told so, the compiler keeps
+// the accumulators in VGPRs; left alone it takes AGPRs and, for fold()'s VALU
+// sums, a copy of each: 2 x 4 blocks then need 180 to 220 registers instead of 151
+// to 166, two waves per SIMD instead of three.  A 16 x 16 tile has registers
+// enough, and in VGPRs its sums move through the registers of loads to come (1 x
+// 512 x 6144: 11.4 us against 10.3).
+constexpr int gs_waves(int FM, int FN, int W) {
+    return FM * FN >= 16 ? 2 : FM * FN >= 8 ? (W == 4 ? 3 : 2) : FN == 4 ? 4 : FN == 2 ? 5 : 1;
+}
 template <int FM, int FN, int W, int MODE>
-__global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, const float* __restrict__ B,
+__global__ __launch_bounds__(64 * W, gs_waves(FM, FN, W)) void k_gemms(const float* __restrict__ A, const float* __restrict__ B,
                                                   float* __restrict__ C, const float* __restrict__ bias,
                                                   const float* __restrict__ res, int M, int N, int K,
                                                   int lda, int ldb, int ldc, int ldr, int act, GsConv cv) {
@@ -74,6 +87,7 @@ __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, c
     constexpr bool CONV = MODE != GS_GEMM, TAPS = MODE == GS_TAPS;
     constexpr int TM = 16 * FM, TN = 16 * FN, LDT = TN + 4;
     constexpr int D = FM * FN >= 16 ? 2 : FM * FN >= 4 ? 3 : 4;   // 16-k blocks in flight, as registers allow
+    constexpr bool REGS = FM * FN <= 4;                 // folded sums in registers; larger tiles: in LDS
     constexpr int NO = TM * TN / (64 * W) > 0 ? TM * TN / (64 * W) : 1;   // outputs per thread
     __shared__ float red[W * TM * LDT];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -205,11 +219,67 @@ __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, c
             }
         }
     };
-    f4s acc[FM][FN];
+    f4s acc[FM][FN], sum[REGS ? FM : 1][REGS ? FN : 1];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = f4s{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < FN; ++j) {
+            acc[i][j] = f4s{0.f, 0.f, 0.f, 0.f};
+            if constexpr (REGS) sum[i][j] = acc[i][j];
+        }
+    // The wave's part of LDS: lane l, register e of block (i, j) <-> row
+    // 16 i + 4 (l / 16) + e, column FN (l % 16) + j.  A lane meets its own elements
+    // only, so adding to them needs no barrier.
+    float* const rw = red + wave * (TM * LDT) + 4 * lg * LDT + FN * lr;
+    bool folded = false;
+    auto to_lds = [&]() {
+        if (REGS || !folded) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) {
+                        if constexpr (REGS) rw[(16 * i + e) * LDT + j] = sum[i][j][e] + acc[i][j][e];
+                        else rw[(16 * i + e) * LDT + j] = acc[i][j][e];
+                    }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                asm volatile("" ::: "memory");          // a quarter at a time, as registers allow
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) rw[(16 * i + e) * LDT + j] += acc[i][j][e];
+            }
+        }
+    };
+    auto fold = [&]() {
+        if constexpr (!REGS) {
+            to_lds();
+            folded = true;
+        }
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                if constexpr (REGS) sum[i][j] += acc[i][j];
+                acc[i][j] = f4s{0.f, 0.f, 0.f, 0.f};
+            }
+    };
+    // The wave's whole rounds of D blocks, a fold after every FOLD of them but the
+    // last: with what follows it a chain is 16 blocks at most.
+    constexpr int FOLD = 16 / D - 1;
+    int done = 0;
+    auto rounds = [&](auto round) {
+        const int whole = n / D * D;
+        for (;;) {
+            const int stop = done + FOLD * D < whole ? done + FOLD * D : whole;
+            for (; done < stop; done += D) round();
+            if (done >= whole) break;
+            fold();
+        }
+    };
     auto clear = [&](float (&as)[FM][4], int lf) {      // channels past Cin: the next pixel's floats
 #pragma unroll
         for (int i = 0; i < FM; ++i)
@@ -233,13 +303,13 @@ __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, c
             };
 #pragma unroll
             for (int s = 0; s < D; ++s) load_taps(a[s], b[s], left[s]);
-            int done = 0;
-            for (; done + D <= n; done += D)
+            rounds([&]() {
 #pragma unroll
                 for (int s = 0; s < D; ++s) {
                     step(a[s], b[s], left[s]);
                     load_taps(a[s], b[s], left[s]);
                 }
+            });
 #pragma unroll
             for (int s = 0; s < D - 1; ++s)
                 if (done + s < n) step(a[s], b[s], left[s]);
@@ -247,13 +317,13 @@ __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, c
     } else if (n > 0) {
 #pragma unroll
         for (int s = 0; s < D; ++s) load(a[s], b[s]);
-        int done = 0;
-        for (; done + D <= n; done += D)
+        rounds([&]() {
 #pragma unroll
             for (int s = 0; s < D; ++s) {
                 mul(a[s], b[s]);
                 load(a[s], b[s]);
             }
+        });
 #pragma unroll
         for (int s = 0; s < D - 1; ++s)
             if (done + s < n) mul(a[s], b[s]);
@@ -273,15 +343,7 @@ __global__ __launch_bounds__(64 * W) void k_gemms(const float* __restrict__ A, c
         mul(as, bs);
     }
 
-    // partial tiles through LDS: lane l, register e of block (i, j) <-> row
-    // 16 i + 4 (l / 16) + e, column FN (l % 16) + j; summed in wave order
-    float* const rw = red + wave * (TM * LDT);
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) rw[(16 * i + 4 * lg + e) * LDT + FN * lr + j] = acc[i][j][e];
+    to_lds();                                           // partial tiles, summed in wave order
     __syncthreads();
 #pragma unroll
     for (int o = 0; o < NO; ++o) {
