@@ -400,13 +400,21 @@ int pick(int M, int N, int K, long long cus, float* us) {
 // from two per CU on); k_gemm_f32 with split-K 16 us and little per K (so a
 // K past some 6,000 on a handful of tiles stays there); k_gemm_f32 without it
 // 4 us + the larger of 0.068 K and its padded product at 55 TFLOP/s (3x3 over
-// 100 x 100 x 17 -> 33, 16 images: 64 us against 103 here); F(2,3) wins from about half a 64 x 64 tile per CU on (3x3 14 x 14 x 256:
-// 8 images, 100 tiles, 21.4 against 31.4 us; 12, 148 tiles, 31.7 against 32.4
-// with the filter transform; 16, 196 tiles, 41 against 33).  5 % in favour of
-// the other kernel.
-bool wins(int M, int N, int K, GsAlt alt, float scale = 1.f) {
+// 100 x 100 x 17 -> 33, 16 images: 64 us against 103 here); F(2,3) wins from
+// about half a 64 x 64 tile per CU on (3x3 14 x 14 x 256: 8 images, 100 tiles,
+// 21.4 against 31.4 us; 12, 148 tiles, 31.7 against 32.4 with the filter
+// transform; 16, 196 tiles, 41 against 33).  A loaded model's layer has its
+// transform (WINO_U: F(2,3) alone): there the unit kernel also wins with few input
+// channels, one round of 32 x 64 tiles here costing 5.4 us + 0.0675 per channel
+// against 4.2 to 5 + 0.085 (6 x 28 x 32 x 16 -> 48, the layer in its model: 7.6 us
+// against 8.8; x 24 -> 64, 117 tiles, 9.8 against 10.4; 48 channels 11.1 against
+// 11.0; 64: 13.2 against 12.3; 128: 18.7 against 16.8); with at most a quarter of
+// the CUs or 32 columns smaller tiles make up for it (4 x 16 x 64 x 16 -> 32: 7.5
+// against 6.9).  5 % in favour of the other kernel.
+bool wins(int M, int N, int K, GsAlt alt, int Cin = 0, float scale = 1.f) {
     const long long t = tiles_of(M, N, 64, 64), cus = num_cus();
     if (alt == GsAlt::WINO) return 2 * t <= cus;
+    if (alt == GsAlt::WINO_U) return 2 * t <= cus && (4 * t <= cus || N <= 32 || Cin > 48);
     if (t > 2 * cus && alt != GsAlt::F32) return false;
     const float n = (float)((t + cus - 1) / cus), k = (float)K;
     float other;
@@ -460,7 +468,7 @@ bool convs_wins(const ConvShape& g, int Cout, GsAlt alt) {
     return M > 0 && K > 0 && Cout > 0 && g.KH <= 8 && g.KW <= 8 &&
            (long long)g.N * g.H * g.W * g.Cin * 4 < 0x7fffffffll && K * Cout * 4 < 0x7fffffffll &&
            M < 0x7fffffffll && tiles_of(M, Cout, 16, 16) < 0x7ffffff0ll &&
-           wins((int)M, Cout, (int)K, alt, g.Cin % 16 ? 1.25f : 1.f);   // GS_TAPS: address work per block
+           wins((int)M, Cout, (int)K, alt, g.Cin, g.Cin % 16 ? 1.25f : 1.f);   // GS_TAPS: address work per block
 }
 
 bool convs_f32(const ConvShape& g, const float* in, const float* w, const float* bias, int Cout, float* out,

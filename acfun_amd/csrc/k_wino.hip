@@ -1600,7 +1600,7 @@ bool run_wino23(const float* in, int N, int H, int W, int Cin, const float* w, c
     }
     // the conv routes may multiply few output tiles directly instead
     const ConvShape gd{N, H, W, Cin, 3, 3, 1, 1, H, W};
-    if (direct && c < 0 && convs_wins(gd, Cout, GsAlt::WINO))
+    if (direct && c < 0 && convs_wins(gd, Cout, Upre && plan == 1 ? GsAlt::WINO_U : GsAlt::WINO))
         return convs_f32(gd, in, w, bias, Cout, out, act, s);
     Scratch Uown(Upre ? 0 : (size_t)16 * Cout * Cinp * sizeof(float), s);
     if (!Upre && !Uown.p) return false;
@@ -1702,9 +1702,9 @@ bool winograd_f32(int tile, const float* in, int N, int H, int W, int Cin, const
     return run_wino23(in, N, H, W, Cin, w, bias, Cout, out, act, s, Upre, false);
 }
 
-bool wino23_direct(int N, int H, int W, int Cin, int Cout) {
+bool wino23_direct(int N, int H, int W, int Cin, int Cout, int plan) {
     const ConvShape g{N, H, W, Cin, 3, 3, 1, 1, H, W};
-    return convs_wins(g, Cout, GsAlt::WINO) && !tune_has("w23", std::vector<int>{N, H, W, Cin, Cout}, kW23NC);
+    return convs_wins(g, Cout, plan == 1 ? GsAlt::WINO_U : GsAlt::WINO) && !tune_has("w23", std::vector<int>{N, H, W, Cin, Cout}, kW23NC);
 }
 
 bool winograd_route_f32(int tile, const float* in, int N, int H, int W, int Cin, const float* w,

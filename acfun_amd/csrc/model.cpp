@@ -625,9 +625,9 @@ int run_model(AcfunModel* m, int N, const float* din, float* dout, hipStream_t s
                     // the weights of a loaded model do not change).
                     const float* U = nullptr;
                     if (groups <= 1 && F.p[0] == 3 && F.p[1] == 3 && F.p[3] == 1 && F.p[4] == 1 &&
-                        in.H >= 3 && in.W >= 3 && in.C >= 4 && o.C >= 4 &&
-                        !wino23_direct(N, in.H, in.W, in.C, o.C)) {
-                        const int plan = wino23_plan(N, in.H, in.W, in.C, o.C, x);
+                        in.H >= 3 && in.W >= 3 && in.C >= 4 && o.C >= 4) {
+                        int plan = wino23_plan(N, in.H, in.W, in.C, o.C, x);
+                        if (wino23_direct(N, in.H, in.W, in.C, o.C, plan)) plan = -1;
                         if (plan >= 0 && F.U_plan != plan) {
                             if (F.U) { (void)hipStreamSynchronize(s); hipFree(F.U); F.U = nullptr; }
                             F.U_plan = -1;

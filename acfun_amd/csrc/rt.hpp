@@ -196,7 +196,7 @@ bool conv32_f32(const ConvShape& g, const float* in, const float* w, const float
 // Few output tiles, or operands of any alignment (k_gemms.hip): small tiles
 // whose K range a workgroup's waves split.  gemms_wins / convs_wins say whether
 // the shape is admitted (a convolution: KH and KW <= 8) and this is the faster kernel than `alt`, the one it would otherwise run.
-enum class GsAlt { G32, CONV32, F32, SPLITK, WINO };
+enum class GsAlt { G32, CONV32, F32, SPLITK, WINO, WINO_U };   // WINO_U: with a filter transform kept from before
 bool gemms_wins(int M, int N, int K, int lda, int ldb, GsAlt alt);
 bool gemms_f32(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
                int ldc, const float* bias, int act, hipStream_t s, const float* res = nullptr,
@@ -256,8 +256,9 @@ bool run_wino43(const float* in, int N, int H, int W, int Cin, const float* w, c
 // rationals, so the faster kernel for the shape runs (within the Winograd
 // tolerance of the reference either way).
 // wino23_direct: a 3x3/s1/p1 shape that winograd_route_f32 multiplies directly
-// (few output tiles, no searched choice of unit kernel): no filter transform.
-bool wino23_direct(int N, int H, int W, int Cin, int Cout);
+// (few output tiles, no searched choice of unit kernel) also when the transform
+// for its plan were there: no filter transform.
+bool wino23_direct(int N, int H, int W, int Cin, int Cout, int plan);
 bool winograd_route_f32(int tile, const float* in, int N, int H, int W, int Cin, const float* w,
                         const float* bias, int Cout, float* out, int act, hipStream_t s,
                         const float* Upre = nullptr);
