@@ -423,9 +423,9 @@ TileCfg tuned_f32_tile(int M, int N, int K, int batch, bool* searched) {
     if (batch != 1) return d;
     const std::vector<int> key{M, N, K};
     bool rec = false;
-    const int c = tune_lookup("f32", key, 16, &rec);
+    const int c = tune_lookup(kTuneF32, key, 16, &rec);
     if (rec)
-        tune_record("f32", key, 16, [M, N, K]() -> TuneRunner {
+        tune_record(kTuneF32, key, 16, [M, N, K]() -> TuneRunner {
             const size_t ab = (size_t)M * K * 4, bb = (size_t)K * N * 4, cb = (size_t)M * N * 4;
             if (ab + bb + cb > ((size_t)2 << 30)) return TuneRunner();
             hipStream_t s = lib_stream();

@@ -943,12 +943,12 @@ bool launch_gemm32(int M, int N, int K, const float* A, int lda, const float* B,
                                                          cv.pad, cv.OH, cv.OW}
                                       : std::vector<int>{0, M, N, K};
     bool rec = false;
-    int c = tune_lookup("g32", key, kG32NC, &rec);
+    int c = tune_lookup(kTuneG32, key, kG32NC, &rec);
     if (rec) {
-        tune_record("g32", key, kG32NC, g32_maker<CONV>(M, N, K, cv));
+        tune_record(kTuneG32, key, kG32NC, g32_maker<CONV>(M, N, K, cv));
         if (autotune_wanted()) {
             autotune_run();
-            c = tune_lookup("g32", key, kG32NC, &rec);
+            c = tune_lookup(kTuneG32, key, kG32NC, &rec);
         }
     }
     if (c < 0 && g32_small<CONV>(M, N, K, lda, ldb, cv))
@@ -996,7 +996,7 @@ namespace acfun {
 void gemm32_register(int M, int N, int K) {
     const std::vector<int> key{0, M, N, K};
     bool rec = false;
-    if (tune_lookup("g32", key, kG32NC, &rec) < 0 && rec)
-        tune_record("g32", key, kG32NC, g32_maker<false>(M, N, K, G32Conv{}));
+    if (tune_lookup(kTuneG32, key, kG32NC, &rec) < 0 && rec)
+        tune_record(kTuneG32, key, kG32NC, g32_maker<false>(M, N, K, G32Conv{}));
 }
 }  // namespace acfun

@@ -814,8 +814,8 @@ bool launch_i8mm(I8M& p, hipStream_t s) {
     if (!getenv("ACFUN_I8_TILE")) {
         const std::vector<int> key{am, p.M, p.N, p.K, p.H, p.W, p.Cinp, p.KW, p.stride, p.pad, p.OH, p.OW};
         bool rec = false;
-        const int c = tune_lookup("i8mm", key, kI8NC, &rec);
-        if (rec) tune_record("i8mm", key, kI8NC, i8mm_maker(p, am));
+        const int c = tune_lookup(kTuneI8mm, key, kI8NC, &rec);
+        if (rec) tune_record(kTuneI8mm, key, kI8NC, i8mm_maker(p, am));
         if (c >= 0) t = i8mm_cand(c, t.per_cu);
     }
     return launch_i8mm_f32(p, t, am, s);

@@ -1595,8 +1595,8 @@ bool run_wino23(const float* in, int N, int H, int W, int Cin, const float* w, c
     if (plan == 1) {
         const std::vector<int> key{N, H, W, Cin, Cout};
         bool rec = false;
-        c = tune_lookup("w23", key, kW23NC, &rec);
-        if (rec) tune_record("w23", key, kW23NC, w23_maker(N, H, W, Cin, Cout));
+        c = tune_lookup(kTuneW23, key, kW23NC, &rec);
+        if (rec) tune_record(kTuneW23, key, kW23NC, w23_maker(N, H, W, Cin, Cout));
     }
     // the conv routes may multiply few output tiles directly instead
     const ConvShape gd{N, H, W, Cin, 3, 3, 1, 1, H, W};
@@ -1704,7 +1704,7 @@ bool winograd_f32(int tile, const float* in, int N, int H, int W, int Cin, const
 
 bool wino23_direct(int N, int H, int W, int Cin, int Cout, int plan) {
     const ConvShape g{N, H, W, Cin, 3, 3, 1, 1, H, W};
-    return convs_wins(g, Cout, plan == 1 ? GsAlt::WINO_U : GsAlt::WINO) && !tune_has("w23", std::vector<int>{N, H, W, Cin, Cout}, kW23NC);
+    return convs_wins(g, Cout, plan == 1 ? GsAlt::WINO_U : GsAlt::WINO) && !tune_has(kTuneW23, std::vector<int>{N, H, W, Cin, Cout}, kW23NC);
 }
 
 bool winograd_route_f32(int tile, const float* in, int N, int H, int W, int Cin, const float* w,

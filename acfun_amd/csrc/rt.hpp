@@ -405,10 +405,9 @@ bool conv2d_route_f32(const float* in, int N, int H, int W, int Cin, const float
                       int groups, float* out, int act, hipStream_t s,
                       const float* wino_U = nullptr);
 
-// The tile search (tune.cpp).  A kernel family (kind "g32", "i8mm", "w23",
-// "f32") asks tune_lookup for the searched candidate of a shape (key) among its
-// ncand candidates: -1 when the search has not covered (arch, kind, key,
-// ncand), and then *record is set the
+// The tile search (tune.cpp).  A kernel family (a kind) asks tune_lookup for the
+// searched candidate of a shape (key) among its ncand candidates: -1 when the
+// search has not covered (arch, kind, key, ncand), and then *record is set the
 // first time the shape is seen in this process, so that the caller registers
 // it with tune_record: ncand candidates and a maker that, called by the
 // search, allocates scratch operands of the shape and returns a runner that
@@ -420,6 +419,12 @@ int tune_lookup(const char* kind, const std::vector<int>& key, int ncand, bool* 
 bool tune_has(const char* kind, const std::vector<int>& key, int ncand);   // a searched candidate exists
 void tune_record(const char* kind, const std::vector<int>& key, int ncand, TuneMaker maker);
 bool autotune_wanted();         // ACFUN_AUTOTUNE=1: true at the first ask of a process
+// The kinds as the cache file names them.  A number after the dot is raised when
+// the family's built-in choice changes: a candidate was adopted for beating the
+// built-in choice of its time, so one from before is asked for no longer and the
+// shape is searched again.  (2: k_gemms before k_gemm32, k_gemm_f32 and F(2,3); kept
+// choices held 196 x 256 x 1024 at 16.5 us, 4.7 by the built-in one.)
+constexpr const char *kTuneG32 = "g32.2", *kTuneF32 = "f32.2", *kTuneW23 = "w23.2", *kTuneI8mm = "i8mm";
 // The replays fill their fp32 operands with this bit pattern (0.01f), not
 // zeros, so the MFMA units see ordinary data.
 constexpr unsigned kTuneFill = 0x3c23d70au;

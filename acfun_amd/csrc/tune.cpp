@@ -10,6 +10,7 @@
 //   "w23"   the F(2,3) unit kernels: unit width and persistent or one unit per
 //           workgroup;
 //   "f32"   k_gemm_f32 (the unaligned fallback): tile and split-K.
+// In the file a kind carries the version of its built-in choice (rt.hpp).
 // A kernel family asks tune_lookup() for its shape's choice and, the first
 // time a shape is seen in a process, registers it with tune_record() together
 // with a maker that can replay the launch on scratch operands of that shape.

@@ -43,21 +43,21 @@ def test_tile_search_caches_and_keeps_parity(gpu, tmp_path):
 def _forced_cache():
     lines = []
     for c, (M, N, K) in enumerate(R.G32_GEMM):
-        lines.append(f"gfx950 g32 11 0,{M},{N},{K} {c}")
+        lines.append(f"gfx950 g32.2 11 0,{M},{N},{K} {c}")
     for c, (N, H, W, Cin, KH, KW, Cout, s, p) in enumerate(R.G32_CONV):
         OH, OW = oracle.out_hw(H, W, KH, KW, s, p)
-        lines.append(f"gfx950 g32 11 1,{N * OH * OW},{Cout},{KH * KW * Cin},{H},{W},{Cin},{KW},{s},{p},{OH},{OW} {c}")
+        lines.append(f"gfx950 g32.2 11 1,{N * OH * OW},{Cout},{KH * KW * Cin},{H},{W},{Cin},{KW},{s},{p},{OH},{OW} {c}")
     for c, (N, H, W, Cin, KH, KW, Cout, s, p) in enumerate(R.I8):
         OH, OW = oracle.out_hw(H, W, KH, KW, s, p)
         Cinp = (Cin + 15) // 16 * 16
         lines.append(f"gfx950 i8mm 5 {AM_C64},{N * OH * OW},{Cout},{KH * KW * Cinp},{H},{W},{Cinp},{KW},"
                      f"{s},{p},{OH},{OW} {c}")
     for c, N, H, W, Cin, Cout in R.W23:
-        lines.append(f"gfx950 w23 5 {N},{H},{W},{Cin},{Cout} {c}")
+        lines.append(f"gfx950 w23.2 5 {N},{H},{W},{Cin},{Cout} {c}")
     for c, (M, N, K) in enumerate(R.F32):
-        lines.append(f"gfx950 f32 16 {M},{N},{K} {c}")
+        lines.append(f"gfx950 f32.2 16 {M},{N},{K} {c}")
     M, N, K = R.F32_KEPT
-    lines.append(f"gfx950 f32 16 {M},{N},{K} -1")
+    lines.append(f"gfx950 f32.2 16 {M},{N},{K} -1")
     return "\n".join(lines) + "\n"
 
 
@@ -65,3 +65,13 @@ def test_every_candidate_keeps_parity(gpu, tmp_path):
     cache = tmp_path / "forced.txt"
     cache.write_text(_forced_cache())
     _child("forced", cache)
+
+
+def test_choices_of_an_older_built_in_are_not_used(gpu, tmp_path):
+    cache = tmp_path / "stale.txt"
+    (gm, gn, gk), (fm, fn, fk), (N, H, W, Cin, Cout) = R.STALE_G32, R.STALE_F32, R.STALE_W23
+    lines = [f"gfx950 g32 11 0,{gm},{gn},{gk} 0", f"gfx950 f32 16 {fm},{fn},{fk} 12",
+             f"gfx950 w23 5 {N},{H},{W},{Cin},{Cout} 0"]
+    cache.write_text("\n".join(lines) + "\n")
+    _child("stale", cache)
+    assert set(lines) <= set(cache.read_text().split("\n"))

@@ -8,7 +8,11 @@
       (written by the parent) assigns every candidate of every family, and
       checks each result against the oracle: every choice the search can make
       computes the same result, including -1 (the search kept the built-in
-      choice).
+      choice);
+  python tests/tune_replay.py stale   -- runs shapes for which the cache file
+      holds candidates adopted against an older built-in choice, checks that
+      the built-in choice runs, searches, and checks that the new search's
+      choices joined the file.
 
 Prints one line per step and "tune ok" at the end; exits non-zero on failure."""
 import os
@@ -34,6 +38,8 @@ W23 = [(0, 2, 40, 36 + 2 * c, 32, 40) for c in range(4)] + [(4, 3, 7, 7, 64, 32)
       [(c, 3, 18, 20, 24, 32) for c in (2, 3)]                             # cand, N, H, W, Cin, Cout
 F32 = [(70 + c, 36, 301) for c in range(16)]                               # K % 4 != 0 -> k_gemm_f32
 F32_KEPT = (86, 36, 301)         # cached as -1: the search kept the built-in choice
+# stale mode: shapes the built-in choice gives to k_gemms
+STALE_G32, STALE_F32, STALE_W23 = (196, 256, 512), (70, 36, 301), (1, 14, 14, 256, 256)
 
 
 def gemm_case(L, rng, M, N, K):
@@ -94,6 +100,24 @@ def run_all(L, rng, forced):
         check(*gemm_ragged_case(L, rng, M, N, K), GEMM_TOL)
 
 
+def stale(L, rng, cache):
+    N, H, W, Cin, Cout = STALE_W23
+    L.acfun_prof_enable(1)
+    check(*gemm_case(L, rng, *STALE_G32), GEMM_TOL)
+    check(*gemm_ragged_case(L, rng, *STALE_F32), GEMM_TOL)
+    check(*conv_case(L, rng, N, H, W, Cin, 3, 3, Cout, 1, 1), WINO_TOL)
+    ran = {name for _, name in capi.prof_report()[0]}
+    L.acfun_prof_enable(0)
+    print("kernels", ran, flush=True)
+    if ran != {"k_gemms"}:
+        sys.exit(1)
+    L.acfun_autotune()
+    kinds = [ln.split()[1] for ln in open(cache).read().split("\n") if ln.strip()]
+    print("cache kinds", kinds, flush=True)
+    if sorted(kinds) != ["f32", "f32.2", "g32", "g32.2", "w23", "w23.2"]:
+        sys.exit(1)
+
+
 def main():
     mode = sys.argv[1]
     cache = os.environ["ACFUN_TUNE_CACHE"]
@@ -102,6 +126,10 @@ def main():
         print("no gfx950 device:", capi.last_error())
         sys.exit(1)
     rng = np.random.default_rng(7)
+    if mode == "stale":
+        stale(L, rng, cache)
+        print("tune ok", flush=True)
+        return
     if mode == "search":
         run_all(L, rng, False)
         L.acfun_autotune()
@@ -113,7 +141,7 @@ def main():
         kinds = {ln.split()[1] for ln in lines if ln.strip()}
         arches = {ln.split()[0] for ln in lines if ln.strip()}
         print("cache kinds", sorted(kinds), "arches", sorted(arches), flush=True)
-        if not {"g32", "i8mm", "w23", "f32"} <= kinds or arches != {"gfx950"}:
+        if not {"g32.2", "i8mm", "w23.2", "f32.2"} <= kinds or arches != {"gfx950"}:
             sys.exit(1)
         run_all(L, rng, False)            # the searched choices give the same results
     else:
