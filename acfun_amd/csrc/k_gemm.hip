@@ -343,13 +343,14 @@ template <bool CONV>
 bool run(GemmP p, int batch, bool va, bool vb, hipStream_t s, const TileCfg* force = nullptr) {
     if (p.M <= 0 || p.N <= 0) return true;
     bool searched = force != nullptr;
-    TileCfg c = force ? *force : tuned_f32_tile(p.M, p.N, p.K, batch, &searched);
+    ConvShape g{};
+    if (CONV && p.K > 0)
+        g = ConvShape{p.M / (p.OH * p.OW), p.H, p.W, p.Cin, p.K / (p.KW * p.Cin), p.KW, p.stride, p.pad, p.OH, p.OW};
+    TileCfg c = force ? *force : tuned_f32_tile(p.M, p.N, p.K, batch, &searched, CONV && p.K > 0 ? &g : nullptr);
     // k_gemms's tiles, which take any alignment, unless the search chose a tile
     const GsAlt alt = c.split > 1 ? GsAlt::SPLITK : GsAlt::F32;
     if (!searched && batch == 1 && p.K > 0) {
         if (CONV) {
-            const ConvShape g{p.M / (p.OH * p.OW), p.H, p.W, p.Cin, p.K / (p.KW * p.Cin), p.KW,
-                              p.stride, p.pad, p.OH, p.OW};
             if (convs_wins(g, p.N, alt)) return convs_f32(g, p.A, p.B, p.bias, p.N, p.C, p.act, s);
         } else if (gemms_wins(p.M, p.N, p.K, p.lda, p.ldb, alt)) {
             return gemms_f32(p.M, p.N, p.K, p.A, p.lda, p.B, p.ldb, p.C, p.ldc, p.bias, p.act, s);
@@ -387,6 +388,20 @@ bool run(GemmP p, int batch, bool va, bool vb, hipStream_t s, const TileCfg* for
     return check_launch("k_splitk_reduce");
 }
 
+// The implicit GEMM of a convolution; force: with this tile.
+bool run_conv(const ConvShape& g, const float* in, const float* w, const float* bias, int Cout, float* out,
+              int act, hipStream_t s, const TileCfg* force = nullptr) {
+    GemmP p{};
+    p.A = in; p.B = w; p.C = out; p.bias = bias;
+    p.M = g.N * g.OH * g.OW; p.N = Cout; p.K = g.KH * g.KW * g.Cin;
+    p.lda = p.K; p.ldb = Cout; p.ldc = Cout; p.act = act;
+    p.H = g.H; p.W = g.W; p.Cin = g.Cin; p.KW = g.KW; p.stride = g.stride; p.pad = g.pad;
+    p.OH = g.OH; p.OW = g.OW;
+    bool va = (g.Cin % 4 == 0) && aligned16(in);
+    bool vb = (Cout % 4 == 0) && aligned16(w);
+    return run<true>(p, 1, va, vb, s, force);
+}
+
 }  // namespace
 
 TileCfg default_f32_tile(int M, int N, int K, int batch) {
@@ -418,15 +433,21 @@ TileCfg f32_cand(int c) {
     return TileCfg{tiles[c / 4][0], tiles[c / 4][1], splits[c % 4]};
 }
 
-TileCfg tuned_f32_tile(int M, int N, int K, int batch, bool* searched) {
+// conv: the shape of the convolution that runs as this GEMM, or null.  It is part
+// of the key: the built-in choice differs, k_gemms's cost too, and so does what a
+// candidate has to gather.
+TileCfg tuned_f32_tile(int M, int N, int K, int batch, bool* searched, const ConvShape* conv) {
     const TileCfg d = default_f32_tile(M, N, K, batch);
     if (batch != 1) return d;
-    const std::vector<int> key{M, N, K};
+    std::vector<int> key{M, N, K};
+    if (conv)
+        key.insert(key.end(), {conv->H, conv->W, conv->Cin, conv->KW, conv->stride, conv->pad, conv->OH, conv->OW});
     bool rec = false;
     const int c = tune_lookup(kTuneF32, key, 16, &rec);
     if (rec)
-        tune_record(kTuneF32, key, 16, [M, N, K]() -> TuneRunner {
-            const size_t ab = (size_t)M * K * 4, bb = (size_t)K * N * 4, cb = (size_t)M * N * 4;
+        tune_record(kTuneF32, key, 16, [M, N, K, is_conv = conv != nullptr, g = conv ? *conv : ConvShape{}]() -> TuneRunner {
+            const size_t ab = is_conv ? (size_t)g.N * g.H * g.W * g.Cin * 4 : (size_t)M * K * 4;
+            const size_t bb = (size_t)K * N * 4, cb = (size_t)M * N * 4;
             if (ab + bb + cb > ((size_t)2 << 30)) return TuneRunner();
             hipStream_t s = lib_stream();
             auto a = std::make_shared<Scratch>(ab, s);
@@ -436,12 +457,18 @@ TileCfg tuned_f32_tile(int M, int N, int K, int batch, bool* searched) {
                 hipMemsetD32Async((hipDeviceptr_t)b->p, kTuneFill, bb / 4, s) != hipSuccess)
                 return TuneRunner();
             return [=](int cand, hipStream_t st) {
+                const float *pa = a->as<float>(), *pb = b->as<float>();
+                float* pc = cc->as<float>();
                 const TileCfg t = cand < 0 ? default_f32_tile(M, N, K) : f32_cand(cand);
-                if (cand < 0 && gemms_wins(M, N, K, K, N, t.split > 1 ? GsAlt::SPLITK : GsAlt::F32))
-                    return gemms_f32(M, N, K, a->as<float>(), K, b->as<float>(), N, cc->as<float>(), N, nullptr,
-                                     0, st);
-                if (t.split > 1 && K < 256 * t.split) return false;
-                return gemm_f32_cfg(M, N, K, a->as<float>(), b->as<float>(), cc->as<float>(), t, st);
+                if (cand >= 0 && t.split > 1 && K < 256 * t.split) return false;
+                const GsAlt alt = t.split > 1 ? GsAlt::SPLITK : GsAlt::F32;
+                if (is_conv) {
+                    if (cand < 0 && convs_wins(g, N, alt)) return convs_f32(g, pa, pb, nullptr, N, pc, 0, st);
+                    return conv_f32_cfg(g, pa, pb, N, pc, t, st);
+                }
+                if (cand < 0 && gemms_wins(M, N, K, K, N, alt))
+                    return gemms_f32(M, N, K, pa, K, pb, N, pc, N, nullptr, 0, st);
+                return gemm_f32_cfg(M, N, K, pa, pb, pc, t, st);
             };
         });
     if (searched) *searched = c >= 0;
@@ -483,6 +510,11 @@ bool gemm_f32_cfg(int M, int N, int K, const float* A, const float* B, float* C,
     return run<false>(p, 1, va, vb, s, &cfg);
 }
 
+bool conv_f32_cfg(const ConvShape& g, const float* in, const float* w, int Cout, float* out, const TileCfg& cfg,
+                  hipStream_t s) {
+    return run_conv(g, in, w, nullptr, Cout, out, 0, s, &cfg);
+}
+
 bool gemm_f32_batched(int batch, int M, int N, int K, const float* A, long long sA, int lda,
                       const float* B, long long sB, int ldb, float* C, long long sC, int ldc,
                       hipStream_t s) {
@@ -496,20 +528,11 @@ bool gemm_f32_batched(int batch, int M, int N, int K, const float* A, long long 
 
 bool conv_igemm_f32(const ConvShape& g, const float* in, const float* w, const float* bias,
                     int Cout, float* out, int act, hipStream_t s) {
-    int M = g.N * g.OH * g.OW;
-    int K = g.KH * g.KW * g.Cin;
     if (g.KH == 1 && g.KW == 1 && g.stride == 1 && g.pad == 0)
-        return gemm_f32(M, Cout, K, in, g.Cin, w, Cout, out, Cout, bias, act, s);
+        return gemm_f32(g.N * g.OH * g.OW, Cout, g.Cin, in, g.Cin, w, Cout, out, Cout, bias, act, s);
     if (conv32_ok(g, Cout, in, w)) return conv32_f32(g, in, w, bias, Cout, out, act, s);
     if (conv_smallc_ok(g, Cout, in)) return conv_smallc_f32(g, in, w, bias, Cout, out, act, s);
-    GemmP p{};
-    p.A = in; p.B = w; p.C = out; p.bias = bias;
-    p.M = M; p.N = Cout; p.K = K; p.lda = K; p.ldb = Cout; p.ldc = Cout; p.act = act;
-    p.H = g.H; p.W = g.W; p.Cin = g.Cin; p.KW = g.KW; p.stride = g.stride; p.pad = g.pad;
-    p.OH = g.OH; p.OW = g.OW;
-    bool va = (g.Cin % 4 == 0) && aligned16(in);
-    bool vb = (Cout % 4 == 0) && aligned16(w);
-    return run<true>(p, 1, va, vb, s);
+    return run_conv(g, in, w, bias, Cout, out, act, s);
 }
 
 bool round_bf16(const float* in, float* out, size_t n, hipStream_t s) {

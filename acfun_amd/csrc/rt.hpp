@@ -435,8 +435,12 @@ const char* tune_status();
 // k_gemm_f32 tiles (the unaligned fallback).
 struct TileCfg { int bm, bn, split; };
 TileCfg default_f32_tile(int M, int N, int K, int batch = 1);
-TileCfg tuned_f32_tile(int M, int N, int K, int batch = 1, bool* searched = nullptr);
-// Runs one fp32 GEMM with an explicit tile config (used by the tile search).
+TileCfg tuned_f32_tile(int M, int N, int K, int batch = 1, bool* searched = nullptr,
+                       const ConvShape* conv = nullptr);
+// Runs one fp32 GEMM / convolution with an explicit tile config (used by the
+// tile search).
+bool conv_f32_cfg(const ConvShape& g, const float* in, const float* w, int Cout, float* out, const TileCfg& cfg,
+                  hipStream_t s);
 bool gemm_f32_cfg(int M, int N, int K, const float* A, const float* B, float* C,
                   const TileCfg& cfg, hipStream_t s);
 

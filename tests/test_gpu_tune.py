@@ -75,3 +75,10 @@ def test_choices_of_an_older_built_in_are_not_used(gpu, tmp_path):
     cache.write_text("\n".join(lines) + "\n")
     _child("stale", cache)
     assert set(lines) <= set(cache.read_text().split("\n"))
+
+
+def test_conv_and_gemm_choices_are_apart(gpu, tmp_path):
+    cache = tmp_path / "keys.txt"
+    H, W, Cin, KW, Cout, s, p, OH, OW = R.KEYS_CONV
+    cache.write_text(f"gfx950 f32.2 16 {OH * OW},{Cout},{KW * KW * Cin},{H},{W},{Cin},{KW},{s},{p},{OH},{OW} 12\n")
+    _child("keys", cache)

@@ -12,7 +12,9 @@
   python tests/tune_replay.py stale   -- runs shapes for which the cache file
       holds candidates adopted against an older built-in choice, checks that
       the built-in choice runs, searches, and checks that the new search's
-      choices joined the file.
+      choices joined the file;
+  python tests/tune_replay.py keys    -- an unaligned convolution with a cached
+      candidate, and the GEMM with its M, N and K without one.
 
 Prints one line per step and "tune ok" at the end; exits non-zero on failure."""
 import os
@@ -40,6 +42,7 @@ F32 = [(70 + c, 36, 301) for c in range(16)]                               # K %
 F32_KEPT = (86, 36, 301)         # cached as -1: the search kept the built-in choice
 # stale mode: shapes the built-in choice gives to k_gemms
 STALE_G32, STALE_F32, STALE_W23 = (196, 256, 512), (70, 36, 301), (1, 14, 14, 256, 256)
+KEYS_CONV = (17, 17, 7, 3, 10, 2, 1, 9, 9)      # H, W, Cin, KH = KW, Cout, s, p, OH, OW: 81 x 10 x 63
 
 
 def gemm_case(L, rng, M, N, K):
@@ -118,6 +121,25 @@ def stale(L, rng, cache):
         sys.exit(1)
 
 
+def keys(L, rng, cache):
+    H, W, Cin, K, Cout, s, p, OH, OW = KEYS_CONV
+    L.acfun_prof_enable(1)
+    check(*conv_case(L, rng, 1, H, W, Cin, K, K, Cout, s, p), GEMM_TOL)
+    conv = {name for _, name in capi.prof_report()[0]}
+    L.acfun_prof_enable(1)
+    check(*gemm_ragged_case(L, rng, OH * OW, Cout, K * K * Cin), GEMM_TOL)
+    gemm = {name for _, name in capi.prof_report()[0]}
+    L.acfun_prof_enable(0)
+    print("conv", conv, "gemm", gemm, flush=True)
+    if conv != {"k_gemm_f32"} or gemm != {"k_gemms"}:
+        sys.exit(1)
+    L.acfun_autotune()
+    lines = [ln for ln in open(cache).read().split("\n") if ln.strip()]
+    print(lines, flush=True)
+    if len(lines) != 2 or not all(ln.startswith("gfx950 f32.2 16 81,10,63") for ln in lines):
+        sys.exit(1)
+
+
 def main():
     mode = sys.argv[1]
     cache = os.environ["ACFUN_TUNE_CACHE"]
@@ -126,8 +148,8 @@ def main():
         print("no gfx950 device:", capi.last_error())
         sys.exit(1)
     rng = np.random.default_rng(7)
-    if mode == "stale":
-        stale(L, rng, cache)
+    if mode in ("stale", "keys"):
+        (stale if mode == "stale" else keys)(L, rng, cache)
         print("tune ok", flush=True)
         return
     if mode == "search":
