@@ -1552,23 +1552,28 @@ TuneMaker w23_maker(int N, int H, int W, int Cin, int Cout) {
     return [=]() -> TuneRunner {
         const int Cinp = (Cin + 15) / 16 * 16, tH = (H + 1) / 2, tW = (W + 1) / 2;
         const ConvShape g{N, H, W, Cin, 3, 3, 1, 1, H, W};
-        // ub also holds the 9 Cin x Cout weights of the direct convolution
+        const bool direct = convs_wins(g, Cout, GsAlt::WINO);
         const size_t ib = (size_t)N * H * W * Cin * 4, ub = (size_t)16 * Cout * Cinp * 4,
-                     ob = (size_t)N * H * W * Cout * 4;
-        if (ib + ub + ob > ((size_t)2 << 30)) return TuneRunner();
+                     ob = (size_t)N * H * W * Cout * 4, wb = direct ? (size_t)9 * Cin * Cout * 4 : 0;
+        if (ib + ub + ob + wb > ((size_t)2 << 30)) return TuneRunner();
         hipStream_t s = lib_stream();
         auto x = std::make_shared<Scratch>(ib, s);
         auto u = std::make_shared<Scratch>(ub, s);
         auto o = std::make_shared<Scratch>(ob, s);
-        if (!x->p || !u->p || !o->p || hipMemsetD32Async((hipDeviceptr_t)x->p, kTuneFill, ib / 4, s) != hipSuccess ||
-            hipMemsetD32Async((hipDeviceptr_t)u->p, kTuneFill, ub / 4, s) != hipSuccess)
+        auto w = std::make_shared<Scratch>(wb, s);
+        if (!x->p || !u->p || !o->p || (direct && !w->p) ||
+            hipMemsetD32Async((hipDeviceptr_t)x->p, kTuneFill, ib / 4, s) != hipSuccess ||
+            hipMemsetD32Async((hipDeviceptr_t)u->p, kTuneFill, ub / 4, s) != hipSuccess ||
+            (direct && hipMemsetD32Async((hipDeviceptr_t)w->p, kTuneFill, wb / 4, s) != hipSuccess))
             return TuneRunner();
         return [=](int cand, hipStream_t st) {
-            if (cand < 0 && convs_wins(g, Cout, GsAlt::WINO))
-                return convs_f32(g, x->as<float>(), u->as<float>(), nullptr, Cout, o->as<float>(), 0, st);
+            if (cand < 0 && direct)
+                return convs_f32(g, x->as<float>(), w->as<float>(), nullptr, Cout, o->as<float>(), 0, st);
             if (cand < 0)
                 return w23_default(x->as<float>(), u->as<float>(), nullptr, o->as<float>(), N, H, W, Cin,
                                    Cinp, Cout, tH, tW, 0, st);
+            // against the direct convolution a candidate pays for its transform, as a call does
+            if (direct && !wino23_filter_impl(w->as<float>(), Cin, Cout, 1, u->as<float>(), st)) return false;
             bool launched = false;
             if (!w23_launch(cand, x->as<float>(), u->as<float>(), nullptr, o->as<float>(), N, H, W, Cin,
                             Cinp, Cout, tH, tW, 0, st, &launched))

@@ -82,3 +82,7 @@ def test_conv_and_gemm_choices_are_apart(gpu, tmp_path):
     H, W, Cin, KW, Cout, s, p, OH, OW = R.KEYS_CONV
     cache.write_text(f"gfx950 f32.2 16 {OH * OW},{Cout},{KW * KW * Cin},{H},{W},{Cin},{KW},{s},{p},{OH},{OW} 12\n")
     _child("keys", cache)
+
+
+def test_search_counts_the_filter_transform(gpu, tmp_path):
+    _child("calls", tmp_path / "calls.txt")

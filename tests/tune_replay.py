@@ -14,7 +14,10 @@
       the built-in choice runs, searches, and checks that the new search's
       choices joined the file;
   python tests/tune_replay.py keys    -- an unaligned convolution with a cached
-      candidate, and the GEMM with its M, N and K without one.
+      candidate, and the GEMM with its M, N and K without one;
+  python tests/tune_replay.py calls   -- a 3x3 convolution with few channels
+      before and after a search (6.7 us directly; 5.5 us for the unit kernel,
+      8.0 us with the filter transform a call makes).
 
 Prints one line per step and "tune ok" at the end; exits non-zero on failure."""
 import os
@@ -140,6 +143,20 @@ def keys(L, rng, cache):
         sys.exit(1)
 
 
+def calls(L, rng, cache):
+    for searched in (False, True):
+        L.acfun_prof_enable(1)
+        check(*conv_case(L, rng, 6, 28, 32, 16, 3, 3, 48, 1, 1), WINO_TOL)
+        ran = {name for _, name in capi.prof_report()[0]}
+        L.acfun_prof_enable(0)
+        print("kernels", ran, flush=True)
+        if ran != {"k_gemms"}:
+            sys.exit(1)
+        if not searched:
+            L.acfun_autotune()
+            print(open(cache).read(), flush=True)
+
+
 def main():
     mode = sys.argv[1]
     cache = os.environ["ACFUN_TUNE_CACHE"]
@@ -148,8 +165,8 @@ def main():
         print("no gfx950 device:", capi.last_error())
         sys.exit(1)
     rng = np.random.default_rng(7)
-    if mode in ("stale", "keys"):
-        (stale if mode == "stale" else keys)(L, rng, cache)
+    if mode in ("stale", "keys", "calls"):
+        {"stale": stale, "keys": keys, "calls": calls}[mode](L, rng, cache)
         print("tune ok", flush=True)
         return
     if mode == "search":
