@@ -332,9 +332,10 @@ bool bf16_region(int M, int N, int ldb, int K, const float* A, const float* B, f
     // Tile by the time of the busiest CU, us, fitted to the sizes above: a tile
     // costs 0.0040, 0.0090 alone on its CU (eight waves, three stages) or 0.0075
     // beside another (four waves, two workgroups per CU), and 0.0262 per K.
+    const long long cus = num_cus();
     auto per_cu = [&](int b) {
         const long long t = (long long)((M + b - 1) / b) * ((N + b - 1) / b);
-        return (float)((t + num_cus() - 1) / num_cus());
+        return (float)((t + cus - 1) / cus);
     };
     const float n128 = per_cu(128), k = (float)Kp;
     const float t64 = 3.f + per_cu(64) * k * 0.0040f;

@@ -350,11 +350,10 @@ bool run(GemmP p, int batch, bool va, bool vb, hipStream_t s, const TileCfg* for
     // k_gemms's tiles, which take any alignment, unless the search chose a tile
     const GsAlt alt = c.split > 1 ? GsAlt::SPLITK : GsAlt::F32;
     if (!searched && batch == 1 && p.K > 0) {
-        if (CONV) {
-            if (convs_wins(g, p.N, alt)) return convs_f32(g, p.A, p.B, p.bias, p.N, p.C, p.act, s);
-        } else if (gemms_wins(p.M, p.N, p.K, p.lda, p.ldb, alt)) {
-            return gemms_f32(p.M, p.N, p.K, p.A, p.lda, p.B, p.ldb, p.C, p.ldc, p.bias, p.act, s);
-        }
+        const int tile = CONV ? convs_tile(g, p.N, alt) : gemms_tile(p.M, p.N, p.K, p.lda, p.ldb, alt);
+        if (tile >= 0)
+            return CONV ? convs_f32(tile, g, p.A, p.B, p.bias, p.N, p.C, p.act, s)
+                        : gemms_f32(tile, p.M, p.N, p.K, p.A, p.lda, p.B, p.ldb, p.C, p.ldc, p.bias, p.act, s);
     }
     if (batch > 1) c.split = 1;
     int splits = c.split < 1 ? 1 : c.split;
@@ -462,13 +461,12 @@ TileCfg tuned_f32_tile(int M, int N, int K, int batch, bool* searched, const Con
                 const TileCfg t = cand < 0 ? default_f32_tile(M, N, K) : f32_cand(cand);
                 if (cand >= 0 && t.split > 1 && K < 256 * t.split) return false;
                 const GsAlt alt = t.split > 1 ? GsAlt::SPLITK : GsAlt::F32;
-                if (is_conv) {
-                    if (cand < 0 && convs_wins(g, N, alt)) return convs_f32(g, pa, pb, nullptr, N, pc, 0, st);
-                    return conv_f32_cfg(g, pa, pb, N, pc, t, st);
-                }
-                if (cand < 0 && gemms_wins(M, N, K, K, N, alt))
-                    return gemms_f32(M, N, K, pa, K, pb, N, pc, N, nullptr, 0, st);
-                return gemm_f32_cfg(M, N, K, pa, pb, pc, t, st);
+                const int tile = cand >= 0 ? -1 : is_conv ? convs_tile(g, N, alt) : gemms_tile(M, N, K, K, N, alt);
+                if (is_conv)
+                    return tile >= 0 ? convs_f32(tile, g, pa, pb, nullptr, N, pc, 0, st)
+                                     : conv_f32_cfg(g, pa, pb, N, pc, t, st);
+                return tile >= 0 ? gemms_f32(tile, M, N, K, pa, K, pb, N, pc, N, nullptr, 0, st)
+                                 : gemm_f32_cfg(M, N, K, pa, pb, pc, t, st);
             };
         });
     if (searched) *searched = c >= 0;

@@ -897,16 +897,16 @@ ConvShape g32_shape(int M, int K, const G32Conv& cv) {
     return ConvShape{M / (cv.OH * cv.OW), cv.H, cv.W, cv.Cin, K / (cv.KW * cv.Cin), cv.KW, cv.stride, cv.pad,
                      cv.OH, cv.OW};
 }
-// The built-in choice runs k_gemms's small tiles instead.
+// The tile, where the built-in choice runs k_gemms instead, else -1.
 template <bool CONV>
-bool g32_small(int M, int N, int K, int lda, int ldb, const G32Conv& cv) {
-    return CONV ? convs_wins(g32_shape(M, K, cv), N, GsAlt::CONV32) : gemms_wins(M, N, K, lda, ldb, GsAlt::G32);
+int g32_small(int M, int N, int K, int lda, int ldb, const G32Conv& cv) {
+    return CONV ? convs_tile(g32_shape(M, K, cv), N, GsAlt::CONV32) : gemms_tile(M, N, K, lda, ldb, GsAlt::G32);
 }
 template <bool CONV>
-bool g32_run_small(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C, int ldc,
+bool g32_run_small(int tile, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C, int ldc,
                    const float* bias, int act, hipStream_t s, const float* res, int ldr, const G32Conv& cv) {
-    return CONV ? convs_f32(g32_shape(M, K, cv), A, B, bias, N, C, act, s, res, ldr)
-                : gemms_f32(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr);
+    return CONV ? convs_f32(tile, g32_shape(M, K, cv), A, B, bias, N, C, act, s, res, ldr)
+                : gemms_f32(tile, M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr);
 }
 
 template <bool CONV>
@@ -923,8 +923,9 @@ TuneMaker g32_maker(int M, int N, int K, const G32Conv& cv) {
             hipMemsetD32Async((hipDeviceptr_t)b->p, kTuneFill, bbytes / 4, s) != hipSuccess)
             return TuneRunner();
         return [=](int cand, hipStream_t st) {
-            if (cand < 0 && g32_small<CONV>(M, N, K, K, N, cv))             // the built-in choice
-                return g32_run_small<CONV>(M, N, K, a->as<float>(), K, b->as<float>(), N, c->as<float>(), N,
+            const int tile = cand < 0 ? g32_small<CONV>(M, N, K, K, N, cv) : -1;   // the built-in choice
+            if (tile >= 0)
+                return g32_run_small<CONV>(tile, M, N, K, a->as<float>(), K, b->as<float>(), N, c->as<float>(), N,
                                            nullptr, 0, st, nullptr, 0, cv);
             if (cand < 0) cand = g32_index(pick_g32(M, N, K, CONV));
             if (!g32_admits(cand, K, CONV ? (long long)cv.bytes : (long long)M * K * 4, N, 0)) return false;
@@ -951,8 +952,9 @@ bool launch_gemm32(int M, int N, int K, const float* A, int lda, const float* B,
             c = tune_lookup(kTuneG32, key, kG32NC, &rec);
         }
     }
-    if (c < 0 && g32_small<CONV>(M, N, K, lda, ldb, cv))
-        return g32_run_small<CONV>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
+    const int tile = c < 0 ? g32_small<CONV>(M, N, K, lda, ldb, cv) : -1;
+    if (tile >= 0)
+        return g32_run_small<CONV>(tile, M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
     const long long a_bytes = CONV ? (long long)cv.bytes : (long long)M * lda * 4;
     if (c < 0 || !g32_admits(c, K, a_bytes, ldc, ldr)) c = g32_index(pick_g32(M, N, K, CONV));
     if (!g32_admits(c, K, a_bytes, ldc, ldr)) c = 0;

@@ -377,8 +377,8 @@ constexpr int kGsN = sizeof(kGs) / sizeof(kGs[0]);
 
 long long tiles_of(long long M, long long N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
-// (cus: num_cus(), asked once per call -- it is a runtime call each time, and
-// one per entry of this table made the smallest products 0.5 us slower)
+// (cus: num_cus(), a runtime call each time; one per entry of this table made the
+// smallest products 0.5 us slower)
 int pick(int M, int N, int K, long long cus, float* us) {
     int best = 0;
     *us = 1e30f;
@@ -393,7 +393,7 @@ int pick(int M, int N, int K, long long cus, float* us) {
     return best;
 }
 
-// Whether these tiles beat the kernel the shape would otherwise run.  That
+// The tile, if it beats the kernel the shape would otherwise run, else -1.  That
 // kernel's time in us by the same kind of fit: k_gemm32 / k_gemm32p over
 // 64 x 64 tiles (up to one per CU: 4.1 + 0.0183 K with its two K groups from
 // K = 512 on; more: 0.0153 K per tile on the busiest CU, a convolution 0.0178, or 0.0169
@@ -411,20 +411,21 @@ int pick(int M, int N, int K, long long cus, float* us) {
 // 11.0; 64: 13.2 against 12.3; 128: 18.7 against 16.8); with at most a quarter of
 // the CUs or 32 columns smaller tiles make up for it (4 x 16 x 64 x 16 -> 32: 7.5
 // against 6.9).  5 % in favour of the other kernel.
-bool wins(int M, int N, int K, GsAlt alt, int Cin = 0, float scale = 1.f) {
+int tile_if_faster(int M, int N, int K, GsAlt alt, int Cin = 0, float scale = 1.f) {
     const long long t = tiles_of(M, N, 64, 64), cus = num_cus();
-    if (alt == GsAlt::WINO) return 2 * t <= cus;
-    if (alt == GsAlt::WINO_U) return 2 * t <= cus && (4 * t <= cus || N <= 32 || Cin > 48);
-    if (t > 2 * cus && alt != GsAlt::F32) return false;
+    const bool wino = alt == GsAlt::WINO || alt == GsAlt::WINO_U;
+    if (wino ? 2 * t > cus : t > 2 * cus && alt != GsAlt::F32) return -1;
+    if (alt == GsAlt::WINO_U && 4 * t > cus && N > 32 && Cin <= 48) return -1;
+    float us;
+    const int tile = pick(M, N, K, cus, &us);
+    if (wino) return tile;
     const float n = (float)((t + cus - 1) / cus), k = (float)K;
     float other;
     if (alt == GsAlt::SPLITK) other = 16.f + 0.0002f * k;
     else if (alt == GsAlt::F32) other = 4.f + fmaxf(0.068f * k, (float)t * k * (2.f * 64 * 64 / 55e6f));
     else if (t <= cus) other = K >= 512 ? 4.1f + 0.0183f * k : 5.5f + 0.0177f * k;
     else other = 4.2f + n * k * (alt == GsAlt::G32 ? 0.0153f : t < 2 * cus ? 0.0178f : 0.0169f);
-    float us;
-    pick(M, N, K, cus, &us);
-    return us * scale < 0.95f * other;
+    return us * scale < 0.95f * other ? tile : -1;
 }
 
 template <int FM, int FN, int W, int MODE>
@@ -438,10 +439,9 @@ bool launch(int M, int N, int K, const float* A, int lda, const float* B, int ld
 }
 
 template <int MODE>
-bool run(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
-                 int ldc, const float* bias, int act, hipStream_t s, const float* res, int ldr, const GsConv& cv) {
-    float us;
-    switch (pick(M, N, K, num_cus(), &us)) {
+bool run(int tile, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
+         int ldc, const float* bias, int act, hipStream_t s, const float* res, int ldr, const GsConv& cv) {
+    switch (tile) {
         case 0: return launch<1, 1, 4, MODE>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
         case 1: return launch<1, 2, 4, MODE>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
         case 2: return launch<1, 4, 4, MODE>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, cv);
@@ -453,32 +453,34 @@ bool run(int M, int N, int K, const float* A, int lda, const float* B, int ldb, 
 
 }  // namespace
 
-bool gemms_wins(int M, int N, int K, int lda, int ldb, GsAlt alt) {
-    return M > 0 && N > 0 && K > 0 && (long long)lda * 64 * 4 < 0x7fffffffll &&
-           (long long)K * ldb * 4 < 0x7fffffffll && tiles_of(M, N, 16, 16) < 0x7ffffff0ll && wins(M, N, K, alt);
+int gemms_tile(int M, int N, int K, int lda, int ldb, GsAlt alt) {
+    const bool fits = M > 0 && N > 0 && K > 0 && (long long)lda * 64 * 4 < 0x7fffffffll &&
+           (long long)K * ldb * 4 < 0x7fffffffll && tiles_of(M, N, 16, 16) < 0x7ffffff0ll;
+    return fits ? tile_if_faster(M, N, K, alt) : -1;
 }
 
-bool gemms_f32(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C, int ldc,
+bool gemms_f32(int tile, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C, int ldc,
                const float* bias, int act, hipStream_t s, const float* res, int ldr) {
-    return run<GS_GEMM>(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, GsConv{});
+    return run<GS_GEMM>(tile, M, N, K, A, lda, B, ldb, C, ldc, bias, act, s, res, ldr, GsConv{});
 }
 
-bool convs_wins(const ConvShape& g, int Cout, GsAlt alt) {
+int convs_tile(const ConvShape& g, int Cout, GsAlt alt) {
     const long long M = (long long)g.N * g.OH * g.OW, K = (long long)g.KH * g.KW * g.Cin;
-    return M > 0 && K > 0 && Cout > 0 && g.KH <= 8 && g.KW <= 8 &&
+    const bool fits = M > 0 && K > 0 && Cout > 0 && g.KH <= 8 && g.KW <= 8 &&
            (long long)g.N * g.H * g.W * g.Cin * 4 < 0x7fffffffll && K * Cout * 4 < 0x7fffffffll &&
-           M < 0x7fffffffll && tiles_of(M, Cout, 16, 16) < 0x7ffffff0ll &&
-           wins((int)M, Cout, (int)K, alt, g.Cin, g.Cin % 16 ? 1.25f : 1.f);   // GS_TAPS: address work per block
+           M < 0x7fffffffll && tiles_of(M, Cout, 16, 16) < 0x7ffffff0ll;
+    // GS_TAPS: address work per block
+    return fits ? tile_if_faster((int)M, Cout, (int)K, alt, g.Cin, g.Cin % 16 ? 1.25f : 1.f) : -1;
 }
 
-bool convs_f32(const ConvShape& g, const float* in, const float* w, const float* bias, int Cout, float* out,
+bool convs_f32(int tile, const ConvShape& g, const float* in, const float* w, const float* bias, int Cout, float* out,
                int act, hipStream_t s, const float* res, int ldr) {
     const GsConv cv{g.H, g.W, g.Cin, g.KW, g.stride, g.pad, g.OH, g.OW,
                     (unsigned)((long long)g.N * g.H * g.W * g.Cin * 4)};
     const int M = g.N * g.OH * g.OW, K = g.KH * g.KW * g.Cin;
     if (g.Cin % 16 == 0)
-        return run<GS_CONV>(M, Cout, K, in, g.Cin, w, Cout, out, Cout, bias, act, s, res, ldr, cv);
-    return run<GS_TAPS>(M, Cout, K, in, g.Cin, w, Cout, out, Cout, bias, act, s, res, ldr, cv);
+        return run<GS_CONV>(tile, M, Cout, K, in, g.Cin, w, Cout, out, Cout, bias, act, s, res, ldr, cv);
+    return run<GS_TAPS>(tile, M, Cout, K, in, g.Cin, w, Cout, out, Cout, bias, act, s, res, ldr, cv);
 }
 
 }  // namespace acfun

@@ -1235,8 +1235,9 @@ bool dwconv_pool_f32(const float* in, int N, int H, int W, int C, const float* w
         // 18 x 58 x 17 x 16 19.5 / 8.2 us, 1 x 112 x 112 x 64 19.7 / 8.5,
         // 8 x 112 x 112 x 96 24.8 / 14.2, 4 x 60 x 90 x 200 23.9 / 11.2.
         const long long row = (PW * C4 + 63) / 64 * 64;
+        const long long full = 2ll * 4 * 64 * num_cus();
         int rp = 4;
-        while (rp > 1 && (long long)N * ((PH + rp - 1) / rp) * row < 2ll * 4 * 64 * num_cus()) --rp;
+        while (rp > 1 && (long long)N * ((PH + rp - 1) / rp) * row < full) --rp;
         const int nstrip = (PH + rp - 1) / rp;
         const long long lanes = (long long)N * nstrip * row;
         const long long wgs = (lanes + 63) / 64;

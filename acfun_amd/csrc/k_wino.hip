@@ -1552,7 +1552,8 @@ TuneMaker w23_maker(int N, int H, int W, int Cin, int Cout) {
     return [=]() -> TuneRunner {
         const int Cinp = (Cin + 15) / 16 * 16, tH = (H + 1) / 2, tW = (W + 1) / 2;
         const ConvShape g{N, H, W, Cin, 3, 3, 1, 1, H, W};
-        const bool direct = convs_wins(g, Cout, GsAlt::WINO);
+        const int tile = convs_tile(g, Cout, GsAlt::WINO);
+        const bool direct = tile >= 0;
         const size_t ib = (size_t)N * H * W * Cin * 4, ub = (size_t)16 * Cout * Cinp * 4,
                      ob = (size_t)N * H * W * Cout * 4, wb = direct ? (size_t)9 * Cin * Cout * 4 : 0;
         if (ib + ub + ob + wb > ((size_t)2 << 30)) return TuneRunner();
@@ -1568,7 +1569,7 @@ TuneMaker w23_maker(int N, int H, int W, int Cin, int Cout) {
             return TuneRunner();
         return [=](int cand, hipStream_t st) {
             if (cand < 0 && direct)
-                return convs_f32(g, x->as<float>(), w->as<float>(), nullptr, Cout, o->as<float>(), 0, st);
+                return convs_f32(tile, g, x->as<float>(), w->as<float>(), nullptr, Cout, o->as<float>(), 0, st);
             if (cand < 0)
                 return w23_default(x->as<float>(), u->as<float>(), nullptr, o->as<float>(), N, H, W, Cin,
                                    Cinp, Cout, tH, tW, 0, st);
@@ -1605,8 +1606,9 @@ bool run_wino23(const float* in, int N, int H, int W, int Cin, const float* w, c
     }
     // the conv routes may multiply few output tiles directly instead
     const ConvShape gd{N, H, W, Cin, 3, 3, 1, 1, H, W};
-    if (direct && c < 0 && convs_wins(gd, Cout, Upre && plan == 1 ? GsAlt::WINO_U : GsAlt::WINO))
-        return convs_f32(gd, in, w, bias, Cout, out, act, s);
+    const int tile = direct && c < 0 ? convs_tile(gd, Cout, Upre && plan == 1 ? GsAlt::WINO_U : GsAlt::WINO) : -1;
+    if (tile >= 0)
+        return convs_f32(tile, gd, in, w, bias, Cout, out, act, s);
     Scratch Uown(Upre ? 0 : (size_t)16 * Cout * Cinp * sizeof(float), s);
     if (!Upre && !Uown.p) return false;
     const float* Up = Upre ? Upre : Uown.as<float>();
@@ -1709,7 +1711,7 @@ bool winograd_f32(int tile, const float* in, int N, int H, int W, int Cin, const
 
 bool wino23_direct(int N, int H, int W, int Cin, int Cout, int plan) {
     const ConvShape g{N, H, W, Cin, 3, 3, 1, 1, H, W};
-    return convs_wins(g, Cout, plan == 1 ? GsAlt::WINO_U : GsAlt::WINO) && !tune_has(kTuneW23, std::vector<int>{N, H, W, Cin, Cout}, kW23NC);
+    return convs_tile(g, Cout, plan == 1 ? GsAlt::WINO_U : GsAlt::WINO) >= 0 && !tune_has(kTuneW23, std::vector<int>{N, H, W, Cin, Cout}, kW23NC);
 }
 
 bool winograd_route_f32(int tile, const float* in, int N, int H, int W, int Cin, const float* w,

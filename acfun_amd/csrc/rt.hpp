@@ -194,15 +194,16 @@ bool conv32_ok(const ConvShape& g, int Cout, const float* in, const float* w);
 bool conv32_f32(const ConvShape& g, const float* in, const float* w, const float* bias, int Cout,
                 float* out, int act, hipStream_t s, const float* res = nullptr, int ldr = 0);
 // Few output tiles, or operands of any alignment (k_gemms.hip): small tiles
-// whose K range a workgroup's waves split.  gemms_wins / convs_wins say whether
-// the shape is admitted (a convolution: KH and KW <= 8) and this is the faster kernel than `alt`, the one it would otherwise run.
+// whose K range a workgroup's waves split.  gemms_tile / convs_tile: the tile to
+// run a shape on where it is admitted (a convolution: KH and KW <= 8) and this is
+// the faster kernel than `alt`, the one it would otherwise run, else -1.
 enum class GsAlt { G32, CONV32, F32, SPLITK, WINO, WINO_U };   // WINO_U: with a filter transform kept from before
-bool gemms_wins(int M, int N, int K, int lda, int ldb, GsAlt alt);
-bool gemms_f32(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
+int gemms_tile(int M, int N, int K, int lda, int ldb, GsAlt alt);
+bool gemms_f32(int tile, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
                int ldc, const float* bias, int act, hipStream_t s, const float* res = nullptr,
                int ldr = 0);
-bool convs_wins(const ConvShape& g, int Cout, GsAlt alt);
-bool convs_f32(const ConvShape& g, const float* in, const float* w, const float* bias, int Cout,
+int convs_tile(const ConvShape& g, int Cout, GsAlt alt);
+bool convs_f32(int tile, const ConvShape& g, const float* in, const float* w, const float* bias, int Cout,
                float* out, int act, hipStream_t s, const float* res = nullptr, int ldr = 0);
 bool gemm_f32(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
               int ldc, const float* bias, int act, hipStream_t s);
