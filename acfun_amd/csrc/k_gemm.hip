@@ -473,6 +473,14 @@ TileCfg tuned_f32_tile(int M, int N, int K, int batch, bool* searched, const Con
     return c >= 0 ? f32_cand(c) : d;
 }
 
+bool fc_splitk() {
+    static const bool on = [] {
+        const char* e = getenv("ACFUN_FC_SPLITK");
+        return !(e && atoi(e) == 0);
+    }();
+    return on;
+}
+
 bool gemm_f32(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
               int ldc, const float* bias, int act, hipStream_t s) {
     GemmP p{};
@@ -487,13 +495,8 @@ bool gemm_f32(int M, int N, int K, const float* A, int lda, const float* B, int 
     // family: k_gemms's tiles up to K of some 6,000, past that the register-
     // staged kernel with K spread over the idle CUs (batch-64 FC 2048 -> 1000:
     // 7.4 us; one tile per CU takes 40.8, split-K with its reduce launch 17.4).
-    // ACFUN_FC_SPLITK=0 turns it off.
-    static const bool fcs = [] {
-        const char* e = getenv("ACFUN_FC_SPLITK");
-        return !(e && atoi(e) == 0);
-    }();
     const long long t64 = (long long)((M + 63) / 64) * ((N + 63) / 64);
-    const bool fc_split = fcs && K >= 1024 && t64 * 4 <= num_cus();
+    const bool fc_split = fc_splitk() && K >= 1024 && t64 * 4 <= num_cus();
     if (K > 0 && !fc_split && gemm32_ok(M, N, K, A, lda, B, ldb))
         return gemm32_f32(M, N, K, A, lda, B, ldb, C, ldc, bias, act, s);
     return run<false>(p, 1, va, vb, s);

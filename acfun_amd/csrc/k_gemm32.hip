@@ -752,6 +752,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 namespace {
 struct G32Tile { int bm, bn, nst, ks = 1, kc = 64, pers = 0; };
 
+// Switches, read once.  ACFUN_G32_KMIN=<K>: the larger tiles from that K on;
+// ACFUN_G32_NOKS: no K groups; ACFUN_G32P=0: no persistent kernel.
+int g32_kmin() {
+    static const int v = [] {
+        const char* e = getenv("ACFUN_G32_KMIN");
+        return e ? atoi(e) : 0x7fffffff;
+    }();
+    return v;
+}
+bool g32_noks() {
+    static const bool v = getenv("ACFUN_G32_NOKS") != nullptr;
+    return v;
+}
+bool g32_pers() {
+    static const bool v = [] {
+        const char* e = getenv("ACFUN_G32P");
+        return !(e && atoi(e) == 0);
+    }();
+    return v;
+}
+
 // Tile choice.  Measured on MI355X (config 1 and the ResNet-50 batch-64
 // layers): 64 x 64 tiles, two or three workgroups per CU, beat the 128-row
 // tiles at every K, since one workgroup per CU leaves the DMA latency and the
@@ -763,29 +784,19 @@ G32Tile pick_g32(int M, int N, int K, bool conv) {
     auto tiles = [&](int bm, int bn) {
         return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
     };
-    // ACFUN_G32_KMIN: the K from which the larger tiles are used (sweeps)
-    static const int kmin = [] {
-        const char* e = getenv("ACFUN_G32_KMIN");
-        return e ? atoi(e) : 0x7fffffff;
-    }();
+    const int kmin = g32_kmin();
     if (K >= kmin && N > 64 && tiles(128, 128) >= cus) return G32Tile{128, 128, 2};
     if (K >= kmin && tiles(128, 64) >= cus) return G32Tile{128, 64, nch > 2 ? 3 : 2};
     // At most one 64 x 64 tile per CU and a long K: two four-wave groups per
     // workgroup split K (two waves per SIMD instead of one).
-    static const bool ks_off = getenv("ACFUN_G32_NOKS") != nullptr;
-    if (!ks_off && nch >= 8 && tiles(64, 64) <= cus) return G32Tile{64, 64, 2, 2};
+    if (!g32_noks() && nch >= 8 && tiles(64, 64) <= cus) return G32Tile{64, 64, 2, 2};
     // More 64 x 64 tiles than CUs: the persistent kernel, two stages, four
     // workgroups per CU.  A GEMM from one tile per CU on (3136 x 512 tiles, 392:
     // K = 64, 256, 512, 2048 take 5.7, 11.6, 19.9, 66.9 us, one tile per
     // workgroup 7.8, 14.7, 23.4, 73.4); a convolution from two (3x3/2 over
     // 14 x 14 x 512, batch 64, 392 tiles: 166 against 160 us -- a tile's pixel
     // set-up is not hidden when most workgroups run a single tile).
-    // ACFUN_G32P=0 turns it off.
-    static const bool pers = [] {
-        const char* e = getenv("ACFUN_G32P");
-        return !(e && atoi(e) == 0);
-    }();
-    if (pers && (conv ? tiles(64, 64) >= 2 * cus : tiles(64, 64) > cus)) return G32Tile{64, 64, 2, 1, 32, 1};
+    if (g32_pers() && (conv ? tiles(64, 64) >= 2 * cus : tiles(64, 64) > cus)) return G32Tile{64, 64, 2, 1, 32, 1};
     // Three stages (one workgroup per CU) only when the tiles fit in one wave;
     // between one and two tiles per CU two stages at two workgroups per CU
     // (config 5's 392-tile layers: GEMM 3136 x 512 x 2048 94.9 -> 81.0 us,
@@ -897,9 +908,13 @@ ConvShape g32_shape(int M, int K, const G32Conv& cv) {
     return ConvShape{M / (cv.OH * cv.OW), cv.H, cv.W, cv.Cin, K / (cv.KW * cv.Cin), cv.KW, cv.stride, cv.pad,
                      cv.OH, cv.OW};
 }
-// The tile, where the built-in choice runs k_gemms instead, else -1.
+// The tile, where the built-in choice runs k_gemms instead, else -1.  Whoever
+// sets a switch of k_gemm32's asks for k_gemm32, and ACFUN_FC_SPLITK=0 for one
+// tile per CU where K would be split.
 template <bool CONV>
 int g32_small(int M, int N, int K, int lda, int ldb, const G32Conv& cv) {
+    if (g32_kmin() != 0x7fffffff || g32_noks() || !g32_pers()) return -1;
+    if (!CONV && !fc_splitk() && K >= 1024 && 4ll * ((M + 63) / 64) * ((N + 63) / 64) <= num_cus()) return -1;
     return CONV ? convs_tile(g32_shape(M, K, cv), N, GsAlt::CONV32) : gemms_tile(M, N, K, lda, ldb, GsAlt::G32);
 }
 template <bool CONV>

@@ -35,6 +35,9 @@
 //   7x7 28 x 28 x 12 -> 224, 9    29.2  (42.4)    3x3 51 x 51 x 143, 60   539   (708)
 #include "rt.hpp"
 
+#include <cstdio>
+#include <cstdlib>
+
 namespace acfun {
 namespace {
 
@@ -393,6 +396,22 @@ int pick(int M, int N, int K, long long cus, float* us) {
     return best;
 }
 
+// ACFUN_GEMMS=0: never; "fm,fn,waves": that tile of kGs for every admitted shape
+// (tests, sweeps).  Read once.
+constexpr int kGsRule = -2, kGsOff = -1;
+int gs_switch() {
+    static const int v = [] {
+        const char* e = getenv("ACFUN_GEMMS");
+        int fm = 0, fn = 0, w = 0;
+        if (!e) return kGsRule;
+        if (sscanf(e, "%d,%d,%d", &fm, &fn, &w) != 3) return atoi(e) == 0 && *e ? kGsOff : kGsRule;
+        for (int i = 0; i < kGsN; ++i)
+            if (kGs[i].fm == fm && kGs[i].fn == fn && kGs[i].w == w) return i;
+        return kGsRule;
+    }();
+    return v;
+}
+
 // The tile, if it beats the kernel the shape would otherwise run, else -1.  That
 // kernel's time in us by the same kind of fit: k_gemm32 / k_gemm32p over
 // 64 x 64 tiles (up to one per CU: 4.1 + 0.0183 K with its two K groups from
@@ -412,6 +431,7 @@ int pick(int M, int N, int K, long long cus, float* us) {
 // the CUs or 32 columns smaller tiles make up for it (4 x 16 x 64 x 16 -> 32: 7.5
 // against 6.9).  5 % in favour of the other kernel.
 int tile_if_faster(int M, int N, int K, GsAlt alt, int Cin = 0, float scale = 1.f) {
+    if (gs_switch() != kGsRule) return gs_switch();
     const long long t = tiles_of(M, N, 64, 64), cus = num_cus();
     const bool wino = alt == GsAlt::WINO || alt == GsAlt::WINO_U;
     if (wino ? 2 * t > cus : t > 2 * cus && alt != GsAlt::F32) return -1;

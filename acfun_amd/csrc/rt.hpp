@@ -205,6 +205,8 @@ bool gemms_f32(int tile, int M, int N, int K, const float* A, int lda, const flo
 int convs_tile(const ConvShape& g, int Cout, GsAlt alt);
 bool convs_f32(int tile, const ConvShape& g, const float* in, const float* w, const float* bias, int Cout,
                float* out, int act, hipStream_t s, const float* res = nullptr, int ldr = 0);
+// ACFUN_FC_SPLITK=0 (false): products with K >= 1024 and few tiles run one tile per CU.
+bool fc_splitk();
 bool gemm_f32(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
               int ldc, const float* bias, int act, hipStream_t s);
 bool conv_igemm_f32(const ConvShape& g, const float* in, const float* w, const float* bias,
