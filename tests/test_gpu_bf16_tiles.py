@@ -12,14 +12,32 @@ from tests.helpers import rel_err
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (16, 16, 1), (80, 144, 128), (144, 80, 129), (272, 528, 640),        # 64
-    (1936, 2064, 384), (1040, 2064, 1100),                               # 128, one per CU
-    (3008, 2000, 300), (2064, 4112, 130),                                # 128, several per CU
-    (4080, 4000, 520), (4112, 3856, 1030),                               # 256
+def tile(torch, M, N, K):
+    """The launcher's choice: 64, "128 alone" on its CU, 128 or 256, by its fit of
+    the busiest CU's time."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    k = -(-K // 128) * 128
+
+    def per_cu(b):
+        return -(-(-(-M // b) * -(-N // b)) // cus)
+
+    n = per_cu(128)
+    us = {64: 3 + per_cu(64) * k * 0.0040, 128: 3 + (k * 0.0090 if n < 2 else n * k * 0.0075),
+          256: 4 + per_cu(256) * k * 0.0262}
+    if us[256] < us[128] and us[256] < us[64]:
+        return 256
+    return 64 if us[64] <= us[128] else "128 alone" if n < 2 else 128
+
+
+@pytest.mark.parametrize("M,N,K,which", [
+    (16, 16, 1, 64), (80, 144, 128, 64), (144, 80, 129, 64), (272, 528, 640, 64),
+    (1040, 2064, 1100, "128 alone"), (1936, 2032, 384, "128 alone"), (1824, 2048, 128, "128 alone"),
+    (1936, 2064, 384, 128), (3008, 2000, 300, 128), (2064, 4112, 130, 128), (4112, 3856, 1030, 128),
+    (4080, 4000, 520, 256), (4080, 3856, 1030, 256), (3856, 4096, 640, 256),
 ])
-def test_bf16_tiles(gpu, rng, M, N, K):
+def test_bf16_tiles(gpu, rng, M, N, K, which):
     torch = pytest.importorskip("torch")
+    assert tile(torch, M, N, K) == which
     g = torch.Generator().manual_seed(int(rng.integers(1 << 30)))
     a, b = (torch.rand(s, generator=g) * 2 - 1 for s in ((M, K), (K, N)))
     ta, tb = a.cuda(), b.cuda()

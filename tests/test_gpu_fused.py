@@ -97,10 +97,10 @@ def test_dw_maxpool_nan_partial_vec(gpu, rng, st):
 
 @pytest.mark.parametrize("C", [16, 20])
 def test_dw_maxpool_nan_strips(gpu, rng, C):
-    """Stride 2 over 3 strips of 4 pooled rows (the row-streaming kernel's
-    unit): NaNs in each strip, at strip boundaries and in the halo rows the
-    strips share, with full (C = 16) and partial (C = 20) max_ps channel
-    groups."""
+    """Stride 2 over 11 strips of one pooled row (the row-streaming kernel's unit
+    for a batch this small; taller ones: test_dw_maxpool_tall_strips): NaNs in
+    and between strips and in the halo rows they share, with full (C = 16) and
+    partial (C = 20) max_ps channel groups."""
     x = rng.standard_normal((2, 41, 22, C)).astype(np.float32)
     for (n, r, c, ch) in ((0, 3, 4, 1), (0, 15, 7, 2), (0, 16, 8, C - 1), (1, 17, 9, 3),
                           (1, 24, 20, C - 2), (0, 31, 0, 0), (1, 33, 21, C - 3), (0, 40, 5, 5)):
@@ -189,10 +189,46 @@ def test_g_maxpool_nan(gpu, rng):
 @pytest.mark.parametrize("N,H,W,C", [(1, 58, 17, 16), (6, 58, 40, 64), (24, 58, 56, 64),
                                      (40, 57, 57, 64), (1, 7, 8, 4)])
 def test_dw_maxpool_strip_heights(gpu, rng, N, H, W, C):
-    """Stride 2 from a handful of lanes to a full chip: strips of 1 to 4 rows."""
+    """Stride 2 from a handful of lanes to a few waves per CU: strips of one pooled row."""
     x = rng.standard_normal((N, H, W, C)).astype(np.float32)
     x[0, H // 2, W // 2, 1] = np.nan
     w = (rng.standard_normal((C, 3, 3)) * 0.3).astype(np.float32)
     b = (rng.standard_normal(C) * 0.1).astype(np.float32)
     assert_bitexact(run_dwpool(gpu, x, w, b, 2, 1, 1, 1, 0), want_dwpool(x, w, b, 2, 1, 1, 1, 0),
                     f"dw+pool {N, H, W, C}")
+
+
+def strip_rows(torch, N, PH, PW, C):
+    """The launcher's pooled rows per strip: fewer than 4 while the lanes do not
+    give each SIMD two waves."""
+    full = 2 * 4 * 64 * torch.cuda.get_device_properties(0).multi_processor_count
+    row = -(-PW * (C // 4) // 64) * 64
+    rp = 4
+    while rp > 1 and N * -(-PH // rp) * row < full:
+        rp -= 1
+    return rp
+
+
+@pytest.mark.parametrize("N,H,W,C,ppad,rp", [
+    (104, 58, 130, 36, 1, 4), (112, 58, 130, 36, 0, 4),      # 15 and 14 pooled rows: a strip of 3, of 2
+    (84, 54, 130, 36, 1, 3), (56, 58, 130, 36, 1, 2),        # 14 by 3, 15 by 2: a strip of 2, of 1
+    (40, 58, 130, 36, 1, 1)])
+def test_dw_maxpool_tall_strips(gpu, rng, N, H, W, C, ppad, rp):
+    """Strips of 1 to 4 pooled rows on a full chip, walked down (even) and up
+    (odd), with a short last strip and a partial max_ps channel group; NaNs at
+    every strip border and in the rows around it, one per image and column."""
+    torch = pytest.importorskip("torch")
+    OH, OW = oracle.out_hw(H, W, 3, 3, 2, 1)
+    PH, PW = oracle.out_hw(OH, OW, 3, 3, 2, ppad)
+    assert strip_rows(torch, N, PH, PW, C) == rp and (rp == 1 or PH % rp)
+    x = rng.standard_normal((N, H, W, C)).astype(np.float32)
+    for n in range(0, N, 2):                       # every other image holds NaNs
+        border = 4 * rp * (1 + n // 2 % max(1, PH // rp))
+        for k, dr in enumerate(range(-5, 6)):
+            if border + dr < H:
+                x[n, border + dr, (7 * n + 11 * k) % W, (n + 5 * k) % C] = np.nan
+    w = (rng.standard_normal((C, 3, 3)) * 0.3).astype(np.float32)
+    b = (rng.standard_normal(C) * 0.1).astype(np.float32)
+    for act, pr in ((0, 0), (1, 1)):
+        assert_bitexact(run_dwpool(gpu, x, w, b, 2, 1, act, ppad, pr),
+                        want_dwpool(x, w, b, 2, 1, act, ppad, pr), f"strips of {rp}, act={act} pr={pr}")

@@ -1,11 +1,12 @@
-"""k_gemms (small tiles, K split between a workgroup's waves, any alignment)
-against the f64 product, at the edges of its tiles and blocks: one row, one
-column, K below, at and just past its 16-deep blocks and their split over the
-waves, rows and columns one past a tile, operands that start 4 bytes past a
-16-byte boundary, and convolutions whose taps change within a wave's run.
-Inputs past the operands are NaN, so a read that leaks into an output shows.
-The bound is fp32 accumulation over K terms, sqrt(K) * 2^-24 on the output's
-scale, taken four times."""
+"""k_gemms (small tiles, K split between a workgroup's waves, any alignment) as
+its rule picks the tile, against the f64 product: one row, one column, K below,
+at and just past its 16-deep blocks and their split over the waves, rows and
+columns one past a tile, GEMM operands that start 4 bytes past a 16-byte
+boundary, and convolutions whose taps change within a wave's run.  (The rule
+picks few of the tiles at these sizes; test_gpu_gemms_forced.py runs each in
+every mode.)  Inputs past the operands are NaN, so a read that leaks into an
+output shows.  The bound is fp32 accumulation over K terms, sqrt(K) * 2^-24 on
+the output's scale, taken four times."""
 import numpy as np
 import pytest
 
