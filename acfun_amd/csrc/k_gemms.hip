@@ -419,7 +419,10 @@ int gs_switch() {
 // from two per CU on); k_gemm_f32 with split-K 16 us and little per K (so a
 // K past some 6,000 on a handful of tiles stays there); k_gemm_f32 without it
 // 4 us + the larger of 0.068 K and its padded product at 55 TFLOP/s (3x3 over
-// 100 x 100 x 17 -> 33, 16 images: 64 us against 103 here); F(2,3) wins from
+// 100 x 100 x 17 -> 33, 16 images: 64 us against 103 here), at 75 TFLOP/s once
+// there are more than six tiles per CU and 64 columns, where its 128 x 128 tiles
+// run in many rounds (3x3/2 over 83 x 65 x 16 -> 224, 33 images, 11 per CU: 55.4 us
+// against 71.3; GEMM 241987 x 259 x 192: 408 against 513); F(2,3) wins from
 // about half a 64 x 64 tile per CU on (3x3 14 x 14 x 256: 8 images, 100 tiles,
 // 21.4 against 31.4 us; 12, 148 tiles, 31.7 against 32.4 with the filter
 // transform; 16, 196 tiles, 41 against 33).  A loaded model's layer has its
@@ -442,7 +445,7 @@ int tile_if_faster(int M, int N, int K, GsAlt alt, int Cin = 0, float scale = 1.
     const float n = (float)((t + cus - 1) / cus), k = (float)K;
     float other;
     if (alt == GsAlt::SPLITK) other = 16.f + 0.0002f * k;
-    else if (alt == GsAlt::F32) other = 4.f + fmaxf(0.068f * k, (float)t * k * (2.f * 64 * 64 / 55e6f));
+    else if (alt == GsAlt::F32) other = 4.f + fmaxf(0.068f * k, (float)t * k * (2.f * 64 * 64 / (t > 6 * cus && N > 64 ? 75e6f : 55e6f)));
     else if (t <= cus) other = K >= 512 ? 4.1f + 0.0183f * k : 5.5f + 0.0177f * k;
     else other = 4.2f + n * k * (alt == GsAlt::G32 ? 0.0153f : t < 2 * cus ? 0.0178f : 0.0169f);
     return us * scale < 0.95f * other ? tile : -1;

@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 import oracle
+from acfun_amd import capi
 from tests.helpers import rel_err
 
 pytestmark = pytest.mark.gpu
@@ -92,3 +93,29 @@ def test_infinities_and_nan_stay_in_their_row(gpu):
     assert bool(torch.isinf(got[7]).all()) and bool(torch.isnan(got[21]).all())
     keep = [i for i in range(M) if i not in (7, 21)]
     assert rel_err(got[keep].numpy(), want[keep].numpy()) < _tol(K)
+
+
+@pytest.mark.parametrize("N,H,W,Cin,ks,Cout,s,kernel", [
+    (33, 83, 65, 16, 3, 224, 2, "k_gemm_f32"),      # 11 tiles of 64 x 64 per CU, K of 144
+    (60, 51, 51, 16, 5, 96, 2, "k_gemms"),          # 5 of them, K of 400
+    (60, 84, 84, 16, 5, 64, 2, "k_gemms"),          # 6.5 of them in one column
+])
+def test_many_tiles_keep_the_faster_kernel(gpu, N, H, W, Cin, ks, Cout, s, kernel):
+    """Large convolutions of few channels: k_gemm_f32's 128 x 128 tiles."""
+    torch = pytest.importorskip("torch")
+    K, p = ks * ks * Cin, ks // 2
+    g = torch.Generator().manual_seed(Cout)
+    x, w = torch.rand((N, H, W, Cin), generator=g), torch.randn((K, Cout), generator=g) / K ** 0.5
+    OH, OW = oracle.out_hw(H, W, ks, ks, s, p)
+    tx, tw, y = x.cuda(), w.cuda(), torch.full((N, OH, OW, Cout), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    gpu.acfun_prof_enable(1)
+    assert gpu.acfun_dev_conv2d(tx.data_ptr(), N, H, W, Cin, tw.data_ptr(), None, ks, ks, Cout, s, p, 1,
+                                y.data_ptr(), 0, None) == 0
+    assert gpu.acfun_sync() == 0
+    ran = {name for _, name in capi.prof_report()[0]}
+    gpu.acfun_prof_enable(0)
+    want = torch.nn.functional.conv2d(x.double().permute(0, 3, 1, 2), w.double().view(ks, ks, Cin, Cout)
+                                      .permute(3, 2, 0, 1), stride=s, padding=p).permute(0, 2, 3, 1)
+    assert rel_err(y.cpu().numpy(), want.numpy()) < _tol(K)
+    assert ran == {kernel}
