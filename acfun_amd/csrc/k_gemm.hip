@@ -438,9 +438,9 @@ TileCfg f32_cand(int c) {
 TileCfg tuned_f32_tile(int M, int N, int K, int batch, bool* searched, const ConvShape* conv) {
     const TileCfg d = default_f32_tile(M, N, K, batch);
     if (batch != 1) return d;
-    std::vector<int> key{M, N, K};
-    if (conv)
-        key.insert(key.end(), {conv->H, conv->W, conv->Cin, conv->KW, conv->stride, conv->pad, conv->OH, conv->OW});
+    const std::vector<int> key = conv ? std::vector<int>{M, N, K, conv->H, conv->W, conv->Cin, conv->KW,
+                                                         conv->stride, conv->pad, conv->OH, conv->OW}
+                                      : std::vector<int>{M, N, K};
     bool rec = false;
     const int c = tune_lookup(kTuneF32, key, 16, &rec);
     if (rec)

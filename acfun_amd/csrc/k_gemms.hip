@@ -422,7 +422,10 @@ int gs_switch() {
 // 100 x 100 x 17 -> 33, 16 images: 64 us against 103 here), at 75 TFLOP/s once
 // there are more than six tiles per CU and 64 columns, where its 128 x 128 tiles
 // run in many rounds (3x3/2 over 83 x 65 x 16 -> 224, 33 images, 11 per CU: 55.4 us
-// against 71.3; GEMM 241987 x 259 x 192: 408 against 513); F(2,3) wins from
+// against 71.3; GEMM 241987 x 259 x 192: 408 against 513); with K up to 32 and 16
+// rows or columns both take less than the host needs for a launch, and that is 0.2
+// us less for k_gemm_f32's one argument (9 x 79 x 16: 3.6 against 3.8; 300 x 300 x
+// 13, past that: 5.1 against 4.2); F(2,3) wins from
 // about half a 64 x 64 tile per CU on (3x3 14 x 14 x 256: 8 images, 100 tiles,
 // 21.4 against 31.4 us; 12, 148 tiles, 31.7 against 32.4 with the filter
 // transform; 16, 196 tiles, 41 against 33).  A loaded model's layer has its
@@ -438,6 +441,7 @@ int tile_if_faster(int M, int N, int K, GsAlt alt, int Cin = 0, float scale = 1.
     const long long t = tiles_of(M, N, 64, 64), cus = num_cus();
     const bool wino = alt == GsAlt::WINO || alt == GsAlt::WINO_U;
     if (wino ? 2 * t > cus : t > 2 * cus && alt != GsAlt::F32) return -1;
+    if (alt == GsAlt::F32 && K <= 32 && (M <= 16 || N <= 16)) return -1;
     if (alt == GsAlt::WINO_U && 4 * t > cus && N > 32 && Cin <= 48) return -1;
     float us;
     const int tile = pick(M, N, K, cus, &us);

@@ -35,9 +35,11 @@ CONVS = [(1, 9, 11, 16, 3, 20, 1, 1), (2, 14, 13, 48, 5, 33, 2, 2), (1, 7, 7, 51
          (1, 9, 8, 1, 3, 5, 2, 1), (2, 13, 11, 3, 5, 17, 2, 2), (1, 14, 9, 5, 4, 7, 3, 0),
          (1, 20, 10, 248, 3, 66, 1, 1), (1, 24, 11, 28, 7, 132, 2, 3), (3, 12, 7, 37, 3, 33, 1, 1),
          (2, 9, 9, 143, 1, 20, 2, 0), (1, 10, 10, 487, 3, 65, 2, 1)]
-# a product, an FC layer, a layer with a tile per CU, a strided and a 3x3/1 convolution
+# a product, an FC layer, a layer with a tile per CU, a strided and a 3x3/1
+# convolution, the smallest unaligned calls and one just past them
 WHICH = {"gemm": (196, 256, 512), "fc": (64, 1000, 2048), "gemm256": (1024, 1024, 1024),
-         "conv": (1, 14, 14, 256, 3, 256, 2, 1), "conv3x3": (1, 14, 14, 256, 3, 256, 1, 1)}
+         "conv": (1, 14, 14, 256, 3, 256, 2, 1), "conv3x3": (1, 14, 14, 256, 3, 256, 1, 1), "tiny": (9, 79, 16), "tiny1x1": (3, 21, 28, 16, 1, 16, 2, 0),
+         "past": (17, 79, 16)}
 
 
 def _tol(K):

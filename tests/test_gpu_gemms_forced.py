@@ -27,7 +27,8 @@ def test_every_tile(tile):
 
 
 @pytest.mark.parametrize("switches,want", [
-    ({}, dict(gemm="k_gemms", fc="k_gemms", gemm256="k_gemms", conv="k_gemms", conv3x3="k_gemms")),
+    ({}, dict(gemm="k_gemms", fc="k_gemms", gemm256="k_gemms", conv="k_gemms", conv3x3="k_gemms",
+              tiny="k_gemm_f32", tiny1x1="k_gemm_f32", past="k_gemms")),
     ({"ACFUN_GEMMS": "0"}, dict(gemm="k_gemm32", fc="k_gemm_f32+k_splitk_reduce", gemm256="k_gemm32",
                                 conv="k_gemm32", conv3x3="k_wino23+k_wino_filter_t")),
     # one tile per CU for the FC layer
