@@ -18,17 +18,20 @@
 // last step's MFMAs cover the barrier and the first reads of the next chunk
 // (64 x 64 tiles, one MFMA per step, read the whole chunk up front).
 //
-// What bounds a large product is LDS: a wave of FM x FN blocks reads
-// 32 (FM + FN) bytes per lane pair for FM x FN MFMAs, and with 64 x 64 tiles (FM
-// = FN = 1) that and the DMA writes take four times the MFMA time.  256 x 256
+// What bounds a large product with small tiles is LDS: a wave of FM x FN blocks
+// reads 32 (FM + FN) bytes per lane pair for FM x FN MFMAs, and with 64 x 64 tiles
+// (FM = FN = 1) that and the DMA writes take four times the MFMA time.  256 x 256
 // tiles on eight 128 x 64 waves bring LDS down to about the MFMA time, at one
-// workgroup per CU; they need 256 tiles to fill the chip.  Measured, us for
-// k_bf16mm alone with 64 x 64 (every size's tile before) / 128 x 128 / 256 x 256:
+// workgroup per CU; they need 256 tiles to fill the chip.  There neither fills the
+// time alone (4096^3: MFMA busy 0.59, LDS reads 0.44 of the cycles, half of them
+// counted as bank conflicts, and the DMA's writes on top).  Measured, us for
+// k_bf16mm alone with 64 x 64 / 128 x 128 / 256 x 256:
 //   4096^3              289 / 127 / 111 (1,234 TFLOP/s)
 //   3008 x 2000 x 4096  109 /  54 /  81
 //   2048^3               41 /  21 /  44
 //   1024^3              6.9 / 11.9 / 25
-// With the packing launch (5.7 TB/s) 4096^3 takes 146 us, 325 before.
+// A whole 4096^3 call, the packing launch (31 us) included, takes 142 to 149 us back
+// to back and 152 with other operands each time; with 64 x 64 tiles 330 and 339.
 #include "rt.hpp"
 
 namespace acfun {
@@ -168,7 +171,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_bf16mm(const unsigned short* _
     const int m0 = (grp * GRP + rin % rows) * BM, n0 = (rin / rows) * BN;
     const int nch = Kp / (KB / 2);
     // quad q of row r sits at slot q ^ sw(r): 8 consecutive rows' reads of one
-    // quad cover all banks
+    // quad take 8 different slots
     auto sw = [](int r) { return QR >= 8 ? r & (QR - 1) : (r >> 1) & (QR - 1); };
     const int sl = lane % QR, rl = lane / QR;
     unsigned av[AIT], bv[BIT];

@@ -25,14 +25,17 @@
 // that crosses the end of a row brings the next row's floats: columns past N
 // are not stored, and the last block clears A's k past K.
 //
-// Measured (us, whole call; before: 64 x 64 tiles, F(2,3), or split-K with a
-// reduce launch):
-//   196 x 256 x 1024 GEMM         4.7   (16.5)    64 x 1000 x 2048 GEMM    7.4  (17.4)
-//   3x3 14 x 14 x 256, 1 image    7.5   (30.2)    3x3 7 x 7 x 512, 1 image 11.5 (59.9)
-//   3x3/2 14 x 14 x 512, 1 image  11.9  (84.0)    999 x 777 x 1333 GEMM    26.9 (57.5)
-//   3x3/2 28 x 28 x 256, 16 imgs  39.2  (47.1)    20001 x 131 x 259 GEMM   36.9 (58.3)
-//   3x3 20 x 20 x 30 -> 50, 2     5.3   (22.1)    3x3 21 x 21 x 248, 1     10.5 (28.7)
-//   7x7 28 x 28 x 12 -> 224, 9    29.2  (42.4)    3x3 51 x 51 x 143, 60   539   (708)
+// Measured (us, whole call; in parentheses with ACFUN_GEMMS=0: 64 x 64 tiles,
+// F(2,3), or split-K with a reduce launch):
+//   196 x 256 x 1024 GEMM         4.7   (14.5)    64 x 1000 x 2048 GEMM    7.0  (16.2)
+//   1024^3 GEMM                  20.6   (22.7)    999 x 777 x 1333 GEMM   26.5  (57.1)
+//   16 x 512 x 6144 GEMM         15.3   (19.4)    20001 x 131 x 259 GEMM  34.1  (57.2)
+//   3x3 14 x 14 x 256, 1 image    7.6   (30.0)    3x3 7 x 7 x 512, 1      11.8  (60.5)
+//   3x3/2 14 x 14 x 512, 1 image 12.4   (84.5)    3x3/2 28 x 28 x 256, 16 40.0  (47.1)
+//   3x3 20 x 20 x 30 -> 50, 2     4.5   (21.7)    3x3 21 x 21 x 248, 1    13.1  (32.8)
+//   7x7 28 x 28 x 12 -> 224, 9   28.9   (42.2)    3x3 51 x 51 x 143, 60  720    (1341)
+// MFMA busy (counters): 0.47 at 1024^3, 0.41 at 999 x 777 x 1333 (208 workgroups),
+// 0.05 to 0.10 in the layers of a model on one image.
 #include "rt.hpp"
 
 #include <cstdio>

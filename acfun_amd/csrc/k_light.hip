@@ -552,9 +552,10 @@ __global__ __launch_bounds__(256) void k_gconv4_3x3(const float* __restrict__ in
 // row y belongs to.  Every value is folded in the reference's order (bias, then
 // one fmaf per in-range tap kh-major; pool taps kh-major, max_ps from -1e30),
 // out-of-range taps skipped by selects, so the result is bit for bit
-// k_dwconv3_blk then k_maxpool3s2_row.  No LDS, no barriers: lanes stream
-// independently, and workgroups are XCD-ordered so the strips that share
-// input rows read them through one L2.  One wave per workgroup: the strips of a
+// k_dwconv3_blk then k_maxpool3s2_row.  No barriers: lanes stream independently
+// (an upward strip keeps its last three depthwise rows in the lane's own part of
+// LDS), and workgroups are XCD-ordered so the strips that share input rows read
+// them through one L2.  One wave per workgroup: the strips of a
 // full chip are some 9.6 waves per CU, which 256-thread workgroups rounded up to
 // 12 on half the CUs (32 x 112 x 112 x 96, inputs in HBM: 43.9 -> 42.7 us; 8
 // images 14.2 -> 13.4).
